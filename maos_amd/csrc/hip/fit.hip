@@ -103,6 +103,38 @@ struct TapT {
     double w;
 };
 
+// A tile of FTX x FTY actuators of one DM, the rows of one wave of kf_mv (lane
+// = column + FTX * row), with all that the wave needs to know of it (one
+// scalar round trip).
+constexpr int FTX = 16, FTY = 4;
+struct FTile {
+    long coef;            // first coefficient
+    int d, ia0, ja0;      // DM and first actuator
+    int a0, anx;          // the first actuator's index, the DM's row length
+    int nx, ny;           // actuators of the tile that exist
+    int eo, cls[5];       // the row's entries: window offsets in FMv::eo, bounds of the four sums
+    int wn, lst;          // window: nodes, their actuators in FMv::list
+    int pitch, own;       // the window's row length, the first actuator's own node
+    int pad_;
+};
+constexpr int FNC = 20;           // coefficients of a row that a wave keeps in registers
+constexpr int FSW = 16;           // most systems per workgroup of kf_mv
+constexpr int FVT = 512;          // threads of kf_vec
+constexpr int FCH = 2 * FVT;      // actuators per workgroup of kf_vec
+// What kf_mv and kf_vec read of a plan, by value (kernel arguments arrive
+// before the first instruction; a record in memory is a round trip away).
+struct FMv {
+    const FTile *tile;
+    const int *list, *eo;
+    const double *coef;       // [tile][entry][64 rows]
+    const double *lr, *lrc;
+    double *r, *p, *p2, *Ap, *b, *part, *res;
+    int *stop;
+    long na, pstride;
+    int nlr, nch, ntile;
+    int o2, o3, o4, o5, o6;
+};
+
 // Everything the kernel reads of one plan (device resident, read through
 // scalar loads as kernel arguments are).
 struct FitDev {
@@ -124,17 +156,32 @@ struct FitDev {
     const int *txp, *typ;
     const TapT *txe, *tye;
     const double *W0, *W1;  // 9 per point (row form), per point
-    const double *NW;       // nact x nnw
     const long *slp, *sli;  // S in CSR (slp null: none)
     const double *slx;
     double tikdiag;
+    // low-rank columns lr [nlr][nact] with coefficients lrc: NW (coefficient
+    // 1) and, with the assembled operator, HA_f' W1 (coefficient -wt_f)
+    int nlr;
+    const double *lr;
+    double lrc[FMAXNW + FMAXFIT];
+    // assembled operator (asm_ok), see kf_mv: row (ia, ja) of DM d1 reaches in
+    // DM d2 (pair d1 * FMAXDM + d2) the kx x ky actuators from (ia + bx, ja + by)
+    // on; its etot[d1] entries over all DMs at epos[ebase[d1]]: column | row <<
+    // 12 | DM << 24
+    const int *epos;
+    int ebase[FMAXDM];
+    int asm_ok, ntile, etot[FMAXDM];
+    int kx[FMAXDM * FMAXDM], ky[FMAXDM * FMAXDM], bx[FMAXDM * FMAXDM], by[FMAXDM * FMAXDM];
+    const struct FTile *tile;
     // launch shape: point chunks of 256 per direction (nc1), actuator chunks
     // of hab actuators x nfit directions (nc3), actuator chunks of 256 (nc4)
     int nc1, nc3, nc4, hab;
+    int nch;  // vector chunks whose partials are kept: of FCH actuators (assembled), else nc4
     // per-system partials, pstride doubles each: W1 . opd_f [nfit][nc1] at
-    // o1, p . Ap [nc3] at o2, NW' p [nnw][nc4] at o3, r . r in two slots
-    // [2][nc4] at o4 (iteration parity), b . b [nc4] at o5
-    int o1, o2, o3, o4, o5;
+    // o1, p . Ap [ntile or nc3] at o2, the low-rank projections [nlr][nch] at
+    // o3, r . r in two slots [2][nch] at o4 (iteration parity), b . b [nch]
+    // at o5, the projections of p in two slots [2][nlr] at o6 (assembled)
+    int o1, o2, o3, o4, o5, o6;
     long pstride;
     // per-system workspace
     double *opd, *opd2;     // [s][nfit][nfloc]
@@ -331,7 +378,7 @@ __global__ __launch_bounds__(FB) void kf_hat(const FitDev *__restrict__ Dp, cons
         for (int q = 0; q < nfit; q++) v += red[j * FB + q * hab + el];
         if (MODE == HAT_L) {
             const double *ps = p + (long)blockIdx.y * na;
-            for (int q = 0; q < D.nnw; q++) v += D.NW[(long)q * na + a] * tnw[q];
+            for (int q = 0; q < D.nnw; q++) v += D.lr[(long)q * na + a] * tnw[q];
             if (D.slp) {
                 double sl = 0;
                 for (long e2 = D.slp[a]; e2 < D.slp[a + 1]; e2++) sl += D.slx[e2] * ps[D.sli[e2]];
@@ -368,8 +415,8 @@ __global__ __launch_bounds__(FB) void kf_init(const FitDev *__restrict__ Dp, dou
         else val = vs[a];
     }
     double *q = fpart(D, s);
-    for (int k = 0; k < D.nnw; k++) {
-        const double c = on ? D.NW[(long)k * na + a] * val : 0.0;
+    for (int k = 0; k < D.nlr; k++) {
+        const double c = on ? D.lr[(long)k * na + a] * val : 0.0;
         const double t = fit_bred(c, wsum);
         if (threadIdx.x == 0) q[D.o3 + k * D.nc4 + blockIdx.x] = t;
         __syncthreads();
@@ -404,9 +451,9 @@ __global__ __launch_bounds__(FB) void kf_restart(const FitDev *__restrict__ Dp, 
     double *q = fpart(D, s);
     const double t = fit_bred(v * v, wsum);
     if (threadIdx.x == 0) q[D.o4 + (k & 1) * D.nc4 + blockIdx.x] = t;
-    for (int j = 0; j < D.nnw; j++) {
+    for (int j = 0; j < D.nlr; j++) {
         __syncthreads();
-        const double c = on ? D.NW[(long)j * na + a] * v : 0.0;
+        const double c = on ? D.lr[(long)j * na + a] * v : 0.0;
         const double u = fit_bred(c, wsum);
         if (threadIdx.x == 0) q[D.o3 + j * D.nc4 + blockIdx.x] = u;
     }
@@ -474,11 +521,434 @@ __global__ __launch_bounds__(FB) void kf_p(const FitDev *__restrict__ Dp, int ws
     }
     double *q = fpart(D, s);
     for (int j = 0; j < D.nnw; j++) {
-        const double c = on ? D.NW[(long)j * na + a] * v : 0.0;
+        const double c = on ? D.lr[(long)j * na + a] * v : 0.0;
         const double u = fit_bred(c, wsum);
         if (threadIdx.x == 0) q[D.o3 + j * D.nc4 + blockIdx.x] = u;
         __syncthreads();
     }
+}
+
+// ---------------------------------------------------------------------------
+// Assembled operator.  HA, W0, S and the Tikhonov term act within a few
+// actuators, so a row of
+//   A = sum_f wt_f HA_f' W0 HA_f + S + tikdiag I
+// is a box of kx x ky actuators of each DM around the row's own position (30 m
+// system: 5 x 5 on its own DM, 7 x 7 on the other), and the rest of FitL is
+// low rank: NW NW' - sum_f wt_f v_f v_f', v_f = HA_f' W1.  The plan holds the
+// box coefficients and the columns NW, v_f, built once on the GPU in FP64.
+// Applying them is one pass with fewer operations than the matrix-free one
+// (about 75 against 106 multiply-adds per actuator) and no fitting-grid arrays
+// in between, and the projections v_f . p follow p's own recurrence, so a CG
+// iteration is two launches (kf_mv, kf_vec) instead of five: for one system
+// of the 30 m fit 12 us of kernels instead of 32 (6 + 6), for 64 systems 43
+// instead of 161 (29 + 14).
+// ---------------------------------------------------------------------------
+
+// Coefficients of the boxes, one thread per (actuator, entry).  Grid (tiles,
+// groups of 4 entries), 256 threads: 4 entries x the 64 actuators of the tile.
+__global__ __launch_bounds__(FB) void kf_assemble(const FitDev *__restrict__ Dp, double *__restrict__ coef) {
+    const FitDev &D = *Dp;
+    const FTile &T = D.tile[blockIdx.x];
+    const int lane = threadIdx.x & 63, d1 = T.d, nd = D.ndm;
+    int e = blockIdx.y * 4 + (threadIdx.x >> 6);
+    if (e >= D.etot[d1]) return;
+    const int ps = D.epos[D.ebase[d1] + e], d2 = ps >> 24;
+    const int pr = d1 * FMAXDM + d2;
+    const int ia = T.ia0 + (lane & (FTX - 1)), ja = T.ja0 + lane / FTX;
+    const int jx = ia + D.bx[pr] + (ps & 0xfff), jy = ja + D.by[pr] + (ps >> 12 & 0xfff);
+    double v = 0;
+    if (ia < D.anx[d1] && ja < D.any[d1] && jx >= 0 && jx < D.anx[d2] && jy >= 0 && jy < D.any[d2]) {
+        const int fnx = D.fnx, fny = D.fny;
+        for (int f = 0; f < D.nfit; f++) {
+            const int px = f * D.tpx + D.tdx[d1] + ia, py = f * D.tpy + D.tdy[d1] + ja;
+            const Tap2 *hx = D.hax + (long)(f * nd + d2) * fnx, *hy = D.hay + (long)(f * nd + d2) * fny;
+            double vf = 0;
+            for (int ey = D.typ[py]; ey < D.typ[py + 1]; ey++)
+                for (int ex = D.txp[px]; ex < D.txp[px + 1]; ex++) {
+                    const TapT ty = D.tye[ey], tx = D.txe[ex];
+                    const double w1 = tx.w * ty.w;
+                    if (!(w1 > FEPS)) continue;
+                    const double *w0 = D.W0 + 9 * ((long)ty.i * fnx + tx.i);
+                    double u = 0;
+                    for (int k = 0; k < 9; k++) {
+                        const int qx = tx.i + k % 3 - 1, qy = ty.i + k / 3 - 1;
+                        if (w0[k] == 0.0 || qx < 0 || qx >= fnx || qy < 0 || qy >= fny) continue;
+                        const Tap2 a = hx[qx], b = hy[qy];
+                        const double wx = a.n == jx ? a.w0 : a.n + 1 == jx ? a.w1 : 0.0;
+                        const double wy = b.n == jy ? b.w0 : b.n + 1 == jy ? b.w1 : 0.0;
+                        const double w2 = wx * wy;
+                        if (w2 > FEPS) u += w0[k] * w2;
+                    }
+                    vf += w1 * u;
+                }
+            v += D.wt[f] * vf;
+        }
+        const long a1 = D.aoff[d1] + (long)ja * D.anx[d1] + ia, a2 = D.aoff[d2] + (long)jy * D.anx[d2] + jx;
+        if (D.slp)
+            for (long q = D.slp[a1]; q < D.slp[a1 + 1]; q++)
+                if (D.sli[q] == a2) v += D.slx[q];
+        if (a1 == a2) v += D.tikdiag;
+    }
+    coef[T.coef + (long)e * 64 + lane] = v;
+}
+
+// v_f = HA_f' W1.  Grid (actuator chunks, directions).
+__global__ __launch_bounds__(FB) void kf_lowrank(const FitDev *__restrict__ Dp, double *__restrict__ out) {
+    const FitDev &D = *Dp;
+    const long a = (long)blockIdx.x * FB + threadIdx.x;
+    const int f = blockIdx.y;
+    if (a >= D.nact) return;
+    int d = 0;
+    while (a >= D.aoff[d + 1]) d++;
+    const int k = (int)(a - D.aoff[d]);
+    const int ja = k / D.anx[d], ia = k - ja * D.anx[d];
+    const int px = f * D.tpx + D.tdx[d] + ia, py = f * D.tpy + D.tdy[d] + ja;
+    double v = 0;
+    for (int ey = D.typ[py]; ey < D.typ[py + 1]; ey++)
+        for (int ex = D.txp[px]; ex < D.txp[px + 1]; ex++) {
+            const double w = D.txe[ex].w * D.tye[ey].w;
+            if (w > FEPS) v += w * D.W1[(long)D.tye[ey].i * D.fnx + D.txe[ex].i];
+        }
+    out[(long)f * D.nact + a] = v;
+}
+
+// Reduces sixteen values per lane over a wave and scatters the sums: lane l
+// ends with value l >> 2, in 17 exchanges instead of 6 per value.
+template <int H, int X>
+__device__ __forceinline__ void red_half(double *u, int lane) {
+    const bool up = (lane & X) != 0;
+#pragma unroll
+    for (int j = 0; j < H; j++) {
+        const double lo = u[j], hi = u[j + H];  // by value: a choice between elements would index memory
+        u[j] = (up ? hi : lo) + __shfl_xor(up ? lo : hi, X, 64);
+    }
+}
+__device__ __forceinline__ double wave_red16(double (&u)[16]) {
+    const int lane = threadIdx.x & 63;
+    red_half<8, 32>(u, lane);
+    red_half<4, 16>(u, lane);
+    red_half<2, 8>(u, lane);
+    red_half<1, 4>(u, lane);
+    double v = u[0];
+    v += __shfl_xor(v, 2, 64);
+    v += __shfl_xor(v, 1, 64);
+    return v;
+}
+
+// out = FitL v.  MV_CG (iteration k): v is the new direction p = r + beta
+// p_old, formed here for the whole window a workgroup reads (each neighbour
+// needs it, so no pass of its own) and stored for the tile's own actuators;
+// its low-rank projections are t = t(r) + beta t_old; partials of p . out per
+// tile.  MV_PLAIN: v is given, its projections are the partials at o3.
+enum { MV_PLAIN = 0, MV_CG = 1 };
+
+// Projections tl[s][j] and beta of S systems from their partials, four lanes
+// per sum, in a fixed order (all threads of the workgroup; no barrier).
+template <int MODE>
+__device__ __forceinline__ void mv_scalars(const FMv &M, int s0, int ns, int k, double (*tl)[FMAXNW + FMAXFIT],
+                                           double *bet) {
+    const int nlr = M.nlr, nch = M.nch, nj = nlr + (MODE == MV_CG ? 1 : 0), sub = threadIdx.x & 3;
+#pragma unroll 2
+    for (int w = threadIdx.x >> 2; w < ns * nj; w += FB / 4) {
+        const int s = w / nj, j = w - s * nj;
+        const double *q = M.part + (long)(s0 + s) * M.pstride;
+        const double *a = j == nlr ? q + M.o4 + (k & 1) * nch : q + M.o3 + j * nch;
+        const double *a2 = q + M.o4 + ((k + 1) & 1) * nch;
+        double u = 0, u2 = 0;
+        for (int i = sub; i < nch; i += 12) {  // three loads each in flight
+            double b[3], b2[3];
+#pragma unroll
+            for (int h = 0; h < 3; h++) {
+                b[h] = a[min(i + 4 * h, nch - 1)];
+                b2[h] = a2[min(i + 4 * h, nch - 1)];
+            }
+#pragma unroll
+            for (int h = 0; h < 3; h++) {
+                u += i + 4 * h < nch ? b[h] : 0.0;
+                u2 += i + 4 * h < nch ? b2[h] : 0.0;
+            }
+        }
+        u += __shfl_xor(u, 2, 64);
+        u2 += __shfl_xor(u2, 2, 64);
+        u += __shfl_xor(u, 1, 64);
+        u2 += __shfl_xor(u2, 1, 64);
+        if (sub == 0) {
+            if (j == nlr) bet[s] = u / u2;
+            else tl[s][j] = u;
+        }
+    }
+}
+// The projections of the new direction (times their coefficients in tl);
+// the first workgroup keeps them for the next iteration.
+template <int MODE>
+__device__ __forceinline__ void mv_project(const FMv &M, int s0, int ns, int k, bool old, bool keep,
+                                           double (*tl)[FMAXNW + FMAXFIT], const double *bet) {
+    const int nlr = M.nlr;
+    for (int w = threadIdx.x; w < ns * 64; w += FB) {
+        const int s = w >> 6, j = w & 63;
+        if (j >= nlr) continue;
+        double u = tl[s][j];
+        if (MODE == MV_CG) {
+            double *q = M.part + (long)(s0 + s) * M.pstride + M.o6;
+            if (old) u += bet[s] * q[((k + 1) & 1) * nlr + j];
+            if (keep) q[(k & 1) * nlr + j] = u;
+        }
+        tl[s][j] = u * M.lrc[j];
+    }
+}
+
+// A workgroup holds a tile of 64 rows, one per lane, for up to FSW systems in
+// turn; its four waves share a row's entries and low-rank columns.  What does
+// not depend on the system stays in registers: a wave's quarter of the
+// coefficients (FNC of them; wider boxes read the rest again) and of the
+// low-rank columns at its rows.  Per system, the window of p (all DMs) goes
+// to LDS, loaded a system ahead, and a box is a sum over entries of a
+// coefficient times the window node at an offset common to the lanes.
+// One system alone (157 workgroups for the 30 m fit) waits for the chain
+// arguments -> tile -> window -> boxes, so whatever does not depend on beta is
+// loaded ahead of it; many systems are bound by the LDS reads, one per
+// multiply-add, and the window loads.  Grid (tiles, padded to a multiple of 8;
+// groups of spw systems); each XCD gets a contiguous run of tiles and finds
+// their coefficients in its own L2.
+template <int MODE>
+__global__ __launch_bounds__(FB, 5) void kf_mv(const FMv M, const double *__restrict__ v, double *__restrict__ out,
+                                             int ws0, int n, int spw, int k, int first) {
+    constexpr int NP = 2;  // window nodes per thread that are loaded ahead
+    constexpr int NLR = 4;  // low-rank columns of a wave that stay in registers
+    extern __shared__ double win[];  // [2][wn]
+    __shared__ double red[2][4][64];
+    __shared__ double tl[FSW][FMAXNW + FMAXFIT], bet[FSW];
+    const int run = gridDim.x >> 3;
+    const int ti = (blockIdx.x & 7) * run + (blockIdx.x >> 3);
+    if (ti >= M.ntile) return;
+    const int g0 = blockIdx.y * spw, ns = min(spw, n - g0);
+    const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6);
+    const FTile &T = M.tile[ti];
+    const int wn = T.wn, nlr = M.nlr;
+    const int *lst = M.list + T.lst;
+    const long na = M.na;
+    double *pn = (k & 1) ? M.p2 : M.p;
+    const double *po = (k & 1) ? M.p : M.p2;
+    const double *src = MODE == MV_PLAIN ? v : M.r;
+    const bool old = MODE == MV_CG && !first;
+    const long sb = (long)((MODE == MV_CG ? ws0 : 0) + g0) * na;
+    int wa[NP];
+    double wu[NP], wp[NP];
+#pragma unroll
+    for (int i = 0; i < NP; i++) {
+        wa[i] = lst[min(t + i * FB, wn - 1)];
+        wu[i] = src[sb + wa[i]];
+        wp[i] = old ? po[sb + wa[i]] : 0.0;
+    }
+    const int c0 = T.cls[wv], nc = T.cls[wv + 1] - c0;
+    const double *cf = M.coef + T.coef + (long)c0 * 64 + lane;
+    const int *eo = M.eo + T.eo + c0;
+    const int eol = eo[min(lane, max(nc - 1, 0))];  // window offsets of the first entries, one per lane
+    double c[FNC];
+#pragma unroll
+    for (int e = 0; e < FNC; e++) {
+        const double ce = cf[e * 64];
+        c[e] = e < nc ? ce : 0.0;
+    }
+    const int ix = lane & (FTX - 1), iy = lane / FTX;
+    const bool on = ix < T.nx && iy < T.ny;
+    const long a = T.a0 + (long)min(iy, T.ny - 1) * T.anx + min(ix, T.nx - 1);
+    const double *lrp = M.lr + a;
+    double cl[NLR];
+#pragma unroll
+    for (int j = 0; j < NLR; j++) cl[j] = lrp[(long)min(wv + 4 * j, nlr - 1) * na];
+    mv_scalars<MODE>(M, ws0 + g0, ns, k, tl, bet);
+    __syncthreads();
+    mv_project<MODE>(M, ws0 + g0, ns, k, old, ti == 0, tl, bet);
+    const int nd0 = iy * T.pitch + ix, own = T.own + nd0;
+    for (int s = 0; s < ns; s++) {
+        const long so = sb + (long)s * na;
+        double *wb = win + (s & 1) * wn;
+        const double be = MODE == MV_CG ? bet[s] : 0.0;
+#pragma unroll
+        for (int i = 0; i < NP; i++)
+            if (t + i * FB < wn) wb[t + i * FB] = old ? be * wp[i] + wu[i] : wu[i];
+        for (int w = t + NP * FB; w < wn; w += FB) {
+            const int b = lst[w];
+            const double u = src[so + b];
+            wb[w] = old ? be * po[so + b] + u : u;
+        }
+        if (s + 1 < ns)
+#pragma unroll
+            for (int i = 0; i < NP; i++) {  // the next system's window
+                wu[i] = src[so + na + wa[i]];
+                wp[i] = old ? po[so + na + wa[i]] : 0.0;
+            }
+        __syncthreads();
+        const double *wr = wb + nd0;
+        double acc = 0;
+#pragma unroll
+        for (int e = 0; e < FNC; e++) acc += c[e] * wr[__builtin_amdgcn_readlane(eol, e)];
+        for (int e = FNC; e < nc; e++) acc += cf[(long)e * 64] * wr[eo[e]];
+#pragma unroll
+        for (int j = 0; j < NLR; j++)
+            if (wv + 4 * j < nlr) acc += cl[j] * tl[s][wv + 4 * j];
+        for (int j = wv + 4 * NLR; j < nlr; j += 4) acc += lrp[(long)j * na] * tl[s][j];
+        red[s & 1][wv][lane] = acc;
+        __syncthreads();
+        if (wv != (s & 3)) continue;
+        // the waves finish systems in turn
+        const double(*q)[64] = red[s & 1];
+        const double y = ((q[0][lane] + q[1][lane]) + q[2][lane]) + q[3][lane];
+        if (on) out[so + a] = y;
+        if (MODE == MV_CG) {
+            const double pv = wb[own];
+            if (on) pn[so + a] = pv;
+            double pap = on ? pv * y : 0.0;
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) pap += __shfl_down(pap, o, 64);
+            if (lane == 0) M.part[(long)(ws0 + g0 + s) * M.pstride + M.o2 + ti] = pap;
+        }
+    }
+}
+
+// Vector passes of the assembled solve, FCH actuators per workgroup (few
+// partials, since every kf_mv workgroup sums them again), two per thread:
+//   VEC_STEP   iteration k, second half: alpha = rr_k / p.Ap; x += alpha p;
+//              r -= alpha Ap; partials of r . r into slot (k + 1) & 1 and of
+//              the projections of r.  A non-finite alpha stops the system (x
+//              keeps its value, the residual is NaN);
+//   VEC_COLD   cold start: x = 0, r = b, stop = 0, partials of b . b, of r . r
+//              (slot 0) and of the projections of r;
+//   VEC_WARM   warm start: stop = 0, partials of b . b and the projections of x;
+//   VEC_PROJ   the projections of x;
+//   VEC_RESTART r = b - Ap, partials of r . r into slot k & 1 and of its
+//              projections.
+// All loads, the low-rank columns among them, are issued before alpha is
+// known: one system alone waits for one round trip and two reductions.
+// x: per-system vectors of stride nact from the launch's first system.  Grid
+// (chunks, systems).
+enum { VEC_STEP, VEC_COLD, VEC_WARM, VEC_PROJ, VEC_RESTART };
+template <int MODE>
+__global__ __launch_bounds__(FVT) void kf_vec(const FMv M, double *__restrict__ x, int ws0, int k) {
+    constexpr int NE = FCH / FVT, NW = FVT / 64;
+    __shared__ double psh[NW][2];
+    __shared__ double sums[16][NW + 1];
+    const int s = ws0 + blockIdx.y, t = threadIdx.x, lane = t & 63, wv = t >> 6;
+    double *q = M.part + (long)s * M.pstride;
+    const long na = M.na;
+    const int nlr = M.nlr, nch = M.nch;
+    const int stopped = MODE == VEC_STEP ? M.stop[s] : 0;
+    long ac[NE];
+    bool on[NE];
+#pragma unroll
+    for (int i = 0; i < NE; i++) {
+        const long a = (long)blockIdx.x * FCH + i * FVT + t;
+        on[i] = a < na;
+        ac[i] = on[i] ? a : na - 1;
+    }
+    const long base = (long)s * na, xb = (long)blockIdx.y * na;
+    double w[NE], bv[NE], pv[NE], ap[NE], xv[NE];  // w: the vector that is projected
+    double c[16][NE];
+#pragma unroll
+    for (int i = 0; i < NE; i++) {
+        w[i] = bv[i] = pv[i] = ap[i] = xv[i] = 0;
+        if (MODE == VEC_STEP) {
+            pv[i] = ((k & 1) ? M.p2 : M.p)[base + ac[i]];
+            w[i] = M.r[base + ac[i]];
+        }
+        if (MODE == VEC_STEP || MODE == VEC_RESTART) ap[i] = M.Ap[base + ac[i]];
+        if (MODE == VEC_COLD || MODE == VEC_WARM || MODE == VEC_RESTART) bv[i] = M.b[base + ac[i]];
+        if (MODE == VEC_STEP || MODE == VEC_WARM || MODE == VEC_PROJ) xv[i] = x[xb + ac[i]];
+    }
+#pragma unroll
+    for (int j = 0; j < 16; j++)
+#pragma unroll
+        for (int i = 0; i < NE; i++) c[j][i] = M.lr[(long)max(min(j, nlr - 1), 0) * na + ac[i]];
+    if (MODE == VEC_STEP) {
+        double rr = 0, pap = 0;
+        for (int i = t; i < nch; i += FVT) rr += q[M.o4 + (k & 1) * nch + i];
+        for (int i = t; i < M.ntile; i += FVT) pap += q[M.o2 + i];
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            rr += __shfl_down(rr, o, 64);
+            pap += __shfl_down(pap, o, 64);
+        }
+        if (lane == 0) {
+            psh[wv][0] = rr;
+            psh[wv][1] = pap;
+        }
+        __syncthreads();
+        rr = pap = 0;
+#pragma unroll
+        for (int i = 0; i < NW; i++) {
+            rr += psh[i][0];
+            pap += psh[i][1];
+        }
+        const double ak = rr / pap;
+        if (stopped || !isfinite(ak)) {
+            if (!stopped && blockIdx.x == 0 && t == 0) {
+                M.stop[s] = 1;
+                M.res[s] = NAN;
+            }
+            return;
+        }
+#pragma unroll
+        for (int i = 0; i < NE; i++) {
+            w[i] = on[i] ? w[i] - ak * ap[i] : 0.0;
+            if (on[i]) {
+                x[xb + ac[i]] = xv[i] + ak * pv[i];
+                M.r[base + ac[i]] = w[i];
+            }
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < NE; i++) {
+            w[i] = MODE == VEC_COLD ? bv[i] : MODE == VEC_RESTART ? bv[i] - ap[i] : xv[i];
+            if (!on[i]) w[i] = bv[i] = 0;
+            if (MODE == VEC_COLD && on[i]) x[xb + ac[i]] = 0;
+            if ((MODE == VEC_COLD || MODE == VEC_RESTART) && on[i]) M.r[base + ac[i]] = w[i];
+        }
+        if ((MODE == VEC_COLD || MODE == VEC_WARM) && blockIdx.x == 0 && t == 0) M.stop[s] = 0;
+    }
+    // sums of the nlr projections, of w . w and of b . b, sixteen at a time
+    for (int j0 = 0; j0 < nlr + 2; j0 += 16) {
+        double u[16];
+#pragma unroll
+        for (int j = 0; j < 16; j++) {
+            u[j] = 0;
+#pragma unroll
+            for (int i = 0; i < NE; i++) {
+                const double wi = w[i], bi = bv[i];
+                double cj = c[j][i];
+                if (j0) cj = M.lr[(long)max(min(j0 + j, nlr - 1), 0) * na + ac[i]];
+                if (j0 + j == nlr) cj = wi;
+                u[j] += j0 + j > nlr ? bi * bi : cj * wi;
+            }
+        }
+        const double v = wave_red16(u);
+        if (j0) __syncthreads();  // the previous sixteen are read
+        if ((lane & 3) == 0) sums[lane >> 2][wv] = v;
+        __syncthreads();
+        const int j = j0 + t;
+        if (t < 16 && j < nlr + 2) {
+            double z = 0;
+#pragma unroll
+            for (int i = 0; i < NW; i++) z += sums[t][i];
+            const int slot = MODE == VEC_STEP ? (k + 1) & 1 : MODE == VEC_RESTART ? k & 1 : 0;
+            if (j < nlr) q[M.o3 + j * nch + blockIdx.x] = z;
+            else if (j == nlr && (MODE == VEC_STEP || MODE == VEC_COLD || MODE == VEC_RESTART))
+                q[M.o4 + slot * nch + blockIdx.x] = z;
+            else if (j == nlr + 1 && (MODE == VEC_COLD || MODE == VEC_WARM)) q[M.o5 + blockIdx.x] = z;
+        }
+    }
+}
+
+// Residual sqrt(r.r / b.b) after the last iteration k.  One workgroup per system.
+__global__ __launch_bounds__(FB) void kf_res(const FitDev *__restrict__ Dp, int ws0, int k) {
+    const FitDev &D = *Dp;
+    __shared__ double psh[4];
+    const int s = ws0 + blockIdx.x;
+    if (D.stop[s]) return;
+    const double *q = fpart(D, s);
+    const double rr = psum(q + D.o4 + ((k + 1) & 1) * D.nch, D.nch, psh);
+    const double bb = psum(q + D.o5, D.nch, psh);
+    if (threadIdx.x == 0) D.res[s] = sqrt(rr / bb);
 }
 
 // Forward taps of one axis: output coordinates u_k (in source grid units).
@@ -511,9 +981,15 @@ struct gpu_fit {
     DBuf<Tap2> hax, hay, hxx, hxy;
     DBuf<int> txp, typ;
     DBuf<TapT> txe, tye;
-    DBuf<double> W0, W1, NW, slx;
+    DBuf<double> W0, W1, slx;
     DBuf<long> slp, sli;
-    DBuf<double> opd, opd2, tnw, r, p, Ap, b, part, res, x;
+    DBuf<double> lr, coef;
+    FMv M{};  // assembled operator
+    int wmax = 0;  // largest window
+    DBuf<int> list, eo, epos;
+    DBuf<FTile> tile;
+    DBuf<double> lrc;
+    DBuf<double> opd, opd2, tnw, r, p, p2, Ap, b, part, res, x;
     DBuf<int> stop;
     DBuf<float> xin;
     std::vector<float> hstage;
@@ -549,6 +1025,164 @@ int fguarded(F &&f) {
         mt::set_error(e.what());
         return MT_EINVAL;
     }
+}
+
+// The assembled operator is used up to this mean box (entries of a row over all
+// DMs): an entry costs about 0.3 us per iteration of 32 systems of the 30 m
+// fit, a direction of the matrix-free passes 11 us, which also cost three more
+// launches.  Nine directions on a ring, 20 warm iterations, assembled against
+// matrix-free, one system / 32: 15" (about 75 entries) 267 against 663 / 678
+// against 1993 us, 30" (150) 291 / 652, 823 / 2023, 60" (350) 655 / 656,
+// 2265 / 2088, 90" 1093 / 655, 5515 / 2189.
+constexpr int FASM_ENTRIES = 256, FASM_BASE = 64, FASM_PER_DIR = 24;
+// ... and to this much memory for the coefficients.
+constexpr size_t FASM_BYTES = (size_t)1 << 30;
+constexpr int FLDS = 65536;  // LDS of a workgroup without an attribute
+
+// LDS of a kf_mv workgroup besides its windows.
+constexpr size_t MV_STATIC = sizeof(double) * (8 * 64 + FSW * (FMAXNW + FMAXFIT + 1));
+
+// Boxes, tiles and windows of the assembled operator (kf_mv); false when the
+// boxes are too large for it (directions far apart on a high DM).
+bool plan_assembled(gpu_fit *g, const std::vector<Tap2> &hax, const std::vector<Tap2> &hay, const std::vector<int> &txp,
+                    const std::vector<int> &typ, const std::vector<TapT> &txe, const std::vector<TapT> &tye,
+                    const mt_fit_recon_t *F) {
+    FitDev &D = g->H;
+    const int nd = D.ndm;
+    // a row's nodes in DM d2 relative to its own indices: the nodes its taps
+    // reach through W0 along any direction, its slaving entries, itself; one
+    // box per pair, the hull over the rows (a row uses less of it where the
+    // DMs' spacings differ)
+    int lo[2][FMAXDM * FMAXDM], hi[2][FMAXDM * FMAXDM];
+    auto add = [&](int ax, int pr, int a, int j) {
+        lo[ax][pr] = std::min(lo[ax][pr], j - a);
+        hi[ax][pr] = std::max(hi[ax][pr], j - a);
+    };
+    for (int d1 = 0; d1 < nd; d1++)
+        for (int d2 = 0; d2 < nd; d2++)
+            for (int ax = 0; ax < 2; ax++) {
+                const int pr = d1 * FMAXDM + d2;
+                const int n1 = (int)(ax ? F->any[d1] : F->anx[d1]), n2 = (int)(ax ? F->any[d2] : F->anx[d2]);
+                const int fn = ax ? D.fny : D.fnx;
+                const std::vector<Tap2> &h = ax ? hay : hax;
+                const std::vector<int> &tp = ax ? typ : txp;
+                const std::vector<TapT> &te = ax ? tye : txe;
+                const int stride = ax ? D.tpy : D.tpx, base = ax ? D.tdy[d1] : D.tdx[d1];
+                lo[ax][pr] = INT32_MAX;
+                hi[ax][pr] = INT32_MIN;
+                if (d1 == d2) add(ax, pr, 0, 0);
+                for (int a = 0; a < n1; a++)
+                    for (int f = 0; f < D.nfit; f++)
+                        for (int e = tp[f * stride + base + a]; e < tp[f * stride + base + a + 1]; e++)
+                            for (int q = std::max(te[e].i - 1, 0); q <= std::min(te[e].i + 1, fn - 1); q++) {
+                                const Tap2 &t = h[(size_t)(f * nd + d2) * fn + q];
+                                if (t.w0 != 0 && t.n >= 0 && t.n < n2) add(ax, pr, a, t.n);
+                                if (t.w1 != 0 && t.n + 1 >= 0 && t.n + 1 < n2) add(ax, pr, a, t.n + 1);
+                            }
+            }
+    if (F->sl_p) {
+        for (int d1 = 0; d1 < nd; d1++)
+            for (long a = D.aoff[d1]; a < D.aoff[d1 + 1]; a++)
+                for (long e = F->sl_p[a]; e < F->sl_p[a + 1]; e++) {
+                    int d2 = 0;
+                    while (F->sl_i[e] >= D.aoff[d2 + 1]) d2++;
+                    const long k1 = a - D.aoff[d1], k2 = F->sl_i[e] - D.aoff[d2];
+                    const int pr = d1 * FMAXDM + d2;
+                    add(0, pr, (int)(k1 % F->anx[d1]), (int)(k2 % F->anx[d2]));
+                    add(1, pr, (int)(k1 / F->anx[d1]), (int)(k2 / F->anx[d2]));
+                }
+    }
+    double entries = 0;
+    for (int d1 = 0; d1 < nd; d1++) {
+        D.etot[d1] = 0;
+        for (int d2 = 0; d2 < nd; d2++) {
+            const int pr = d1 * FMAXDM + d2;
+            const bool any = lo[0][pr] <= hi[0][pr] && lo[1][pr] <= hi[1][pr];
+            D.bx[pr] = any ? lo[0][pr] : 0;
+            D.by[pr] = any ? lo[1][pr] : 0;
+            D.kx[pr] = any ? hi[0][pr] - lo[0][pr] + 1 : 0;
+            D.ky[pr] = any ? hi[1][pr] - lo[1][pr] + 1 : 0;
+            if ((double)D.kx[pr] * D.ky[pr] > 4096) return false;  // positions are kept in 12 bits
+            D.etot[d1] += D.kx[pr] * D.ky[pr];
+        }
+        entries += (double)D.etot[d1] * (D.aoff[d1 + 1] - D.aoff[d1]);
+    }
+    if (entries > (double)std::min(FASM_ENTRIES, FASM_BASE + FASM_PER_DIR * D.nfit) * D.nact) return false;
+    // entries of a row in the order of the sums: DM, box column, box row; the
+    // four sums take consecutive quarters
+    std::vector<int> epos;
+    for (int d1 = 0; d1 < nd; d1++) {
+        D.ebase[d1] = (int)epos.size();
+        for (int d2 = 0; d2 < nd; d2++)
+            for (int x = 0; x < D.kx[d1 * FMAXDM + d2]; x++)
+                for (int y = 0; y < D.ky[d1 * FMAXDM + d2]; y++) epos.push_back(x | y << 12 | d2 << 24);
+    }
+    // window of a tile: the boxes' nodes in every DM, all at one pitch, so that
+    // an entry is at one offset from every row
+    int pitch[FMAXDM], woff[FMAXDM * FMAXDM], wn[FMAXDM], eob[FMAXDM];
+    std::vector<int> eo;
+    g->wmax = 0;
+    for (int d1 = 0; d1 < nd; d1++) {
+        pitch[d1] = wn[d1] = 0;
+        for (int d2 = 0; d2 < nd; d2++) pitch[d1] = std::max(pitch[d1], FTX - 1 + D.kx[d1 * FMAXDM + d2]);
+        for (int d2 = 0; d2 < nd; d2++) {
+            const int pr = d1 * FMAXDM + d2;
+            woff[pr] = wn[d1];
+            if (D.ky[pr]) wn[d1] += pitch[d1] * (FTY - 1 + D.ky[pr]);
+        }
+        eob[d1] = (int)eo.size();
+        for (int e = 0; e < D.etot[d1]; e++) {
+            const int ps = epos[D.ebase[d1] + e];
+            eo.push_back(woff[d1 * FMAXDM + (ps >> 24)] + (ps >> 12 & 0xfff) * pitch[d1] + (ps & 0xfff));
+        }
+        g->wmax = std::max(g->wmax, wn[d1]);
+    }
+    if (sizeof(double) * 2 * g->wmax + MV_STATIC > FLDS) return false;
+    std::vector<FTile> tile;
+    std::vector<int> list;
+    long coef = 0;
+    for (int d1 = 0; d1 < nd; d1++)
+        for (int ja = 0; ja < D.any[d1]; ja += FTY)
+            for (int ia = 0; ia < D.anx[d1]; ia += FTX) {
+                FTile T{};
+                T.coef = coef;
+                T.d = d1;
+                T.ia0 = ia;
+                T.ja0 = ja;
+                T.anx = D.anx[d1];
+                T.a0 = (int)D.aoff[d1] + ja * D.anx[d1] + ia;
+                T.nx = std::min(FTX, D.anx[d1] - ia);
+                T.ny = std::min(FTY, D.any[d1] - ja);
+                T.eo = eob[d1];
+                for (int q = 0; q <= 4; q++) T.cls[q] = (int)((long)D.etot[d1] * q / 4);
+                T.wn = wn[d1];
+                T.lst = (int)list.size();
+                T.pitch = pitch[d1];
+                T.own = woff[d1 * FMAXDM + d1] - D.by[d1 * FMAXDM + d1] * pitch[d1] - D.bx[d1 * FMAXDM + d1];
+                // nodes outside a DM read any actuator (their coefficients are zero)
+                list.resize(list.size() + wn[d1], T.a0);
+                for (int d2 = 0; d2 < nd; d2++) {
+                    const int pr = d1 * FMAXDM + d2;
+                    for (int y = 0; D.ky[pr] && y < FTY - 1 + D.ky[pr]; y++)
+                        for (int x = 0; x < FTX - 1 + D.kx[pr]; x++) {
+                            const int jx = ia + D.bx[pr] + x, jy = ja + D.by[pr] + y;
+                            if (jx < 0 || jx >= D.anx[d2] || jy < 0 || jy >= D.any[d2]) continue;
+                            list[T.lst + woff[pr] + y * pitch[d1] + x] = (int)D.aoff[d2] + jy * D.anx[d2] + jx;
+                        }
+                }
+                tile.push_back(T);
+                coef += (long)D.etot[d1] * FTX * FTY;
+            }
+    if ((size_t)coef * sizeof(double) > FASM_BYTES || list.size() > (size_t)INT32_MAX) return false;
+    D.ntile = (int)tile.size();
+    g->tile.upload(tile);
+    g->epos.upload(epos);
+    g->list.upload(list);
+    g->eo.upload(eo);
+    g->coef.alloc(coef + FTX * FTY * FNC);  // kf_mv loads FNC entries of any wave
+    D.tile = g->tile.p;
+    D.epos = g->epos.p;
+    return true;
 }
 
 void build_fit_plan(gpu_fit *g, const mt_recon_t *R, const mt_fit_recon_t *F) {
@@ -647,7 +1281,6 @@ void build_fit_plan(gpu_fit *g, const mt_recon_t *R, const mt_fit_recon_t *F) {
     g->tye.upload(tye);
     g->W0.upload(std::vector<double>(F->W0, F->W0 + 9 * D.nfloc));
     g->W1.upload(std::vector<double>(F->W1, F->W1 + D.nfloc));
-    if (D.nnw) g->NW.upload(std::vector<double>(F->NW, F->NW + (size_t)D.nnw * D.nact));
     if (F->sl_p) {
         std::vector<long> p(F->sl_p, F->sl_p + D.nact + 1);
         const long nz = p[D.nact];
@@ -665,17 +1298,24 @@ void build_fit_plan(gpu_fit *g, const mt_recon_t *R, const mt_fit_recon_t *F) {
     D.tye = g->tye.p;
     D.W0 = g->W0.p;
     D.W1 = g->W1.p;
-    D.NW = g->NW.p;
     D.slp = g->slp.p;
     D.sli = g->sli.p;
     D.slx = g->slx.p;
     D.tikdiag = F->tikdiag;
+    D.asm_ok = plan_assembled(g, hax, hay, txp, typ, txe, tye, F) ? 1 : 0;
+    D.nlr = D.nnw + (D.asm_ok ? D.nfit : 0);
+    for (int k = 0; k < D.nlr; k++) D.lrc[k] = k < D.nnw ? 1.0 : -D.wt[k - D.nnw];
+    g->lr.alloc((size_t)D.nlr * D.nact);
+    if (D.nnw)
+        FCHK(hipMemcpy(g->lr.p, F->NW, sizeof(double) * D.nnw * D.nact, hipMemcpyHostToDevice));
+    D.lr = g->lr.p;
     // workspace
     const long ns = g->nbatch;
     g->opd.alloc(ns * D.nfit * D.nfloc);
     g->opd2.alloc(ns * D.nfit * D.nfloc);
     g->r.alloc(ns * D.nact);
     g->p.alloc(ns * D.nact);
+    if (D.asm_ok) g->p2.alloc(ns * D.nact);
     g->Ap.alloc(ns * D.nact);
     g->b.alloc(ns * D.nact);
     g->tnw.alloc(ns * FMAXNW);
@@ -686,10 +1326,12 @@ void build_fit_plan(gpu_fit *g, const mt_recon_t *R, const mt_fit_recon_t *F) {
     D.nc4 = (int)((D.nact + FB - 1) / FB);
     D.o1 = 0;
     D.o2 = D.o1 + D.nfit * D.nc1;
-    D.o3 = D.o2 + D.nc3;
-    D.o4 = D.o3 + D.nnw * D.nc4;
-    D.o5 = D.o4 + 2 * D.nc4;
-    D.pstride = D.o5 + D.nc4;
+    D.nch = D.asm_ok ? (int)((D.nact + FCH - 1) / FCH) : D.nc4;
+    D.o3 = D.o2 + (D.asm_ok ? D.ntile : D.nc3);
+    D.o4 = D.o3 + D.nlr * D.nch;
+    D.o5 = D.o4 + 2 * D.nch;
+    D.o6 = D.o5 + D.nch;
+    D.pstride = D.o6 + (D.asm_ok ? 2 * D.nlr : 0);
     g->part.alloc(ns * D.pstride);
     g->stop.alloc(ns);
     FCHK(hipMemset(g->stop.p, 0, sizeof(int) * ns));
@@ -708,6 +1350,39 @@ void build_fit_plan(gpu_fit *g, const mt_recon_t *R, const mt_fit_recon_t *F) {
     D.res = g->res.p;
     g->dev.alloc(1);
     FCHK(hipMemcpy(g->dev.p, &D, sizeof(FitDev), hipMemcpyHostToDevice));
+    if (D.asm_ok) {
+        FMv &M = g->M;
+        g->lrc.upload(std::vector<double>(D.lrc, D.lrc + D.nlr));
+        M.tile = g->tile.p;
+        M.list = g->list.p;
+        M.eo = g->eo.p;
+        M.coef = g->coef.p;
+        M.lr = D.lr;
+        M.lrc = g->lrc.p;
+        M.r = D.r;
+        M.p = D.p;
+        M.p2 = g->p2.p;
+        M.Ap = D.Ap;
+        M.b = D.b;
+        M.part = D.part;
+        M.res = D.res;
+        M.stop = D.stop;
+        M.na = D.nact;
+        M.pstride = D.pstride;
+        M.nlr = D.nlr;
+        M.nch = D.nch;
+        M.ntile = D.ntile;
+        M.o2 = D.o2;
+        M.o3 = D.o3;
+        M.o4 = D.o4;
+        M.o5 = D.o5;
+        M.o6 = D.o6;
+        const int emax = *std::max_element(D.etot, D.etot + D.ndm);
+        hipLaunchKernelGGL(kf_assemble, dim3(D.ntile, (emax + 3) / 4), dim3(FB), 0, 0, g->dev.p, g->coef.p);
+        hipLaunchKernelGGL(kf_lowrank, dim3(D.nc4, D.nfit), dim3(FB), 0, 0, g->dev.p, g->lr.p + (size_t)D.nnw * D.nact);
+        FCHK(hipGetLastError());
+        FCHK(hipStreamSynchronize(0));
+    }
 }
 
 // Launch sequences.  ws0: first workspace slot; n: systems; external
@@ -716,6 +1391,7 @@ void build_fit_plan(gpu_fit *g, const mt_recon_t *R, const mt_fit_recon_t *F) {
 dim3 grid_pts(const FitDev &D, int n) { return dim3(D.nc1, D.nfit, n); }
 dim3 grid_hat(const FitDev &D, int n) { return dim3(D.nc3, n); }
 dim3 grid_act(const FitDev &D, int n) { return dim3(D.nc4, n); }
+dim3 grid_vec(const FitDev &D, int n) { return dim3(D.nch, n); }  // assembled
 
 // Interpolation from nsrc sources, GS of them per group of loads: 2 for up
 // to two sources, 3 for three, else 4 (a partial last group reloads the
@@ -736,33 +1412,64 @@ void enq_rhs(gpu_fit *g, hipStream_t st, const float *xin, long xstride, double 
     hipLaunchKernelGGL(kf_hat<HAT_R>, grid_hat(D, n), dim3(FB), 0, st, g->dev.p, (const double *)nullptr, out, ws0);
 }
 
-// out = FitL p; the partials of NW' p must be in place (kf_init, kf_restart
-// or kf_p wrote them).
+// FitL of n systems with the assembled operator.
+template <int MODE>
+void launch_mv(gpu_fit *g, hipStream_t st, const double *v, double *out, int ws0, int n, int k, int first) {
+    const int nt = (g->M.ntile + 7) / 8 * 8;
+    // about five workgroups per CU (what its registers hold), each with at
+    // least one system and at most FSW
+    const int groups = std::max(std::min(n, 1280 / nt), (n + FSW - 1) / FSW);
+    const int spw = (n + groups - 1) / groups;
+    hipLaunchKernelGGL((kf_mv<MODE>), dim3(nt, (n + spw - 1) / spw), dim3(FB), sizeof(double) * 2 * g->wmax, st, g->M, v,
+                       out, ws0, n, spw, k, first);
+}
+
+// out = FitL p; the partials of the low-rank projections of p must be in
+// place (kf_init, kf_restart or kf_p wrote them).
 void enq_L(gpu_fit *g, hipStream_t st, const double *p, double *out, int ws0, int n) {
     const FitDev &D = g->H;
+    if (D.asm_ok) {
+        launch_mv<MV_PLAIN>(g, st, p, out, ws0, n, 0, 0);
+        return;
+    }
     launch_fwd<0>(D, D.ndm, grid_pts(D, n), st, g->dev.p, (const void *)p, D.nact, ws0);
     hipLaunchKernelGGL(kf_w, grid_pts(D, n), dim3(FB), 0, st, g->dev.p, ws0, 1);
     hipLaunchKernelGGL(kf_hat<HAT_L>, grid_hat(D, n), dim3(FB), 0, st, g->dev.p, p, out, ws0);
 }
 
 // The whole solve of n systems (lib/pcg.c:28-113 with Mmul = NULL: z = r,
-// restart every 100 iterations): 5 launches per iteration.
+// restart every 100 iterations): 2 launches per iteration with the assembled
+// operator, else 5.
 void enq_solve(gpu_fit *g, hipStream_t st, const float *xin, long xstride, double *x, int ws0, int n, int warm,
                int maxit) {
     const FitDev &D = g->H;
     const long na = D.nact;
     double *b = g->b.p + (long)ws0 * na, *p = g->p.p + (long)ws0 * na, *Ap = g->Ap.p + (long)ws0 * na;
     enq_rhs(g, st, xin, xstride, b, ws0, n);
-    hipLaunchKernelGGL(kf_init<true>, grid_act(D, n), dim3(FB), 0, st, g->dev.p, x, ws0, warm);
+    if (!D.asm_ok) hipLaunchKernelGGL(kf_init<true>, grid_act(D, n), dim3(FB), 0, st, g->dev.p, x, ws0, warm);
+    else if (warm) hipLaunchKernelGGL(kf_vec<VEC_WARM>, grid_vec(D, n), dim3(FVT), 0, st, g->M, x, ws0, 0);
+    else hipLaunchKernelGGL(kf_vec<VEC_COLD>, grid_vec(D, n), dim3(FVT), 0, st, g->M, x, ws0, 0);
     for (int k = 0; k < maxit; k++) {
         if (k % 100 == 0) {
-            if (k == 0 && !warm) {
+            if (D.asm_ok) {
+                if (k > 0) hipLaunchKernelGGL(kf_vec<VEC_PROJ>, grid_vec(D, n), dim3(FVT), 0, st, g->M, x, ws0, k);
+                if (k > 0 || warm) {
+                    enq_L(g, st, x, Ap, ws0, n);
+                    hipLaunchKernelGGL(kf_vec<VEC_RESTART>, grid_vec(D, n), dim3(FVT), 0, st, g->M, x, ws0, k);
+                }
+            } else if (k == 0 && !warm) {
                 hipLaunchKernelGGL(kf_restart<true>, grid_act(D, n), dim3(FB), 0, st, g->dev.p, ws0, k);
             } else {
                 if (k > 0) hipLaunchKernelGGL(kf_init<false>, grid_act(D, n), dim3(FB), 0, st, g->dev.p, x, ws0, 1);
                 enq_L(g, st, x, Ap, ws0, n);
                 hipLaunchKernelGGL(kf_restart<false>, grid_act(D, n), dim3(FB), 0, st, g->dev.p, ws0, k);
             }
+        }
+        if (D.asm_ok) {
+            launch_mv<MV_CG>(g, st, nullptr, g->Ap.p, ws0, n, k, (int)(k % 100 == 0));
+            hipLaunchKernelGGL(kf_vec<VEC_STEP>, grid_vec(D, n), dim3(FVT), 0, st, g->M, x, ws0, k);
+            if (k + 1 == maxit) hipLaunchKernelGGL(kf_res, dim3(n), dim3(FB), 0, st, g->dev.p, ws0, k);
+            continue;
         }
         enq_L(g, st, p, Ap, ws0, n);
         hipLaunchKernelGGL(kf_upd, grid_act(D, n), dim3(FB), 0, st, g->dev.p, x, ws0, k);
@@ -930,7 +1637,10 @@ int gpu_fit_L(gpu_fit_t *g, const double *a, double *out, double alpha, double b
             if (!std::isfinite(a[i])) ffail(MT_ENOTFINITE, "non-finite input vector");
         // the input goes to the p slot of system 0, the output to its r slot
         FCHK(hipMemcpyAsync(g->p.p, a, sizeof(double) * na, hipMemcpyHostToDevice, g->stream));
-        hipLaunchKernelGGL(kf_init<false>, grid_act(g->H, 1), dim3(FB), 0, g->stream, g->dev.p, g->p.p, 0, 1);
+        if (g->H.asm_ok)
+            hipLaunchKernelGGL(kf_vec<VEC_PROJ>, grid_vec(g->H, 1), dim3(FVT), 0, g->stream, g->M, g->p.p, 0, 0);
+        else
+            hipLaunchKernelGGL(kf_init<false>, grid_act(g->H, 1), dim3(FB), 0, g->stream, g->dev.p, g->p.p, 0, 1);
         enq_L(g, g->stream, g->p.p, g->r.p, 0, 1);
         FCHK(hipGetLastError());
         std::vector<double> h(na);

@@ -228,3 +228,46 @@ def test_fit_graph_cache_eviction_in_flight(fitsys):
     for da in outs:
         da.free()
     dx.free()
+
+
+# name: (aperture, directions' ring radius in arcsec, DM spacings, direction
+# heights, systems); sizes at the edges of the apply's tiles (16 x 4
+# actuators, 20 register entries a wave, 16 systems a workgroup)
+ASSEMBLED = {
+    "one_dm": (6.0, 0.0, [0.5], float("inf"), 1),            # box within the registers, partial tiles
+    "spacings": (8.0, 10.0, [0.5, 0.45], float("inf"), 5),   # spacings differ: hull of the rows' boxes
+    "wide": (12.0, 30.0, [0.5, 0.5], float("inf"), 3),       # boxes past the registers
+    "finite": (12.0, 10.0, [0.5, 0.5], 90e3, 18),            # converging directions, more systems than a workgroup holds
+    "matrix_free": (10.0, 120.0, [0.5, 0.5], float("inf"), 3),  # boxes too large: the five-pass form
+}
+
+
+@pytest.mark.parametrize("name", list(ASSEMBLED))
+def test_fit_operator_forms(name):
+    """FitL and the solve of every geometry the assembled operator accepts,
+    and of one it leaves to the matrix-free passes, against the oracle; a
+    system's result is the same bits in every batch.  L: two FP64 orders of
+    the same sums, under 1e3 terms of 1e-16 each (1e-12)."""
+    D, ring, dxs, hs, n = ASSEMBLED[name]
+    base = configs.batch_member(D, 2, 2)
+    th = [(0.0, 0.0, 0.5)] + [(ring * np.cos(t), ring * np.sin(t), 0.125) for t in (0.3, 1.9, 3.2, 5.0)]
+    dms = [dict(ht=11800.0 * k, dx=dx, offset=0.5 * k, guard=1.0, iac=0.0) for k, dx in enumerate(dxs)]
+    fc = configs.fit_for(base, dm=dms, fit=th, fit_hs=[hs] * len(th), fit_maxit=12)
+    r = tomo.Recon(configs.with_fit_dirs(base, fc))
+    f = tomo.FitSetup(r, fc)
+    print("case", name, "nact", f.nact, "nfloc", f.nfloc, flush=True)
+    g, o = tomo.GpuFit(r, f, nbatch=n), FitOracle(r, f, nthread=8)
+    rng = np.random.default_rng(7)
+    a = rng.standard_normal(f.nact)
+    assert rel(g.L(a), o.fit_l(a)) < 1e-12
+    xs = (rng.standard_normal((n, r.nx)) * 1e-7).astype(np.float32)
+    dx, da = DevArray.of(xs), DevArray((n, f.nact), np.float64)
+    g.solve_dev(dx.ptr, da.ptr, nsys=n)
+    sync()
+    got = da.numpy()
+    assert rel(got[n - 1], o.solve(xs[n - 1].astype(np.float64), 12)[0]) < 1e-9
+    for k in range(n):
+        assert np.array_equal(got[k], g.solve(xs[k].astype(np.float64), isys=k)[0]), k
+    g.close()
+    dx.free()
+    da.free()
