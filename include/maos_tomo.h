@@ -421,7 +421,7 @@ int  gpu_tomo_autotune(gpu_tomo_t *g, int nsys, int *choice);
 /* Set the launch shape directly, e.g. to replay an autotuned choice without
  * timing: choice[6] = systems per workgroup of the WFS, layer and LDS
  * column kernels (each 1, 2 or 4, or 0 for the built-in heuristic), the
- * layer tile rows (16, 32, 64, or 0 for 64 where it fits), the column kernel
+ * layer tile rows (16, 32, 64, or 0 for the built-in choice), the column kernel
  * (1 registers where it applies, 2 LDS stages, 0 as 1; 2 also keeps the row
  * FFTs in LDS stages, which otherwise run in registers for single-plan
  * batches with layers of 64 or 96 points) and the flights of a

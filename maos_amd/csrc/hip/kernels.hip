@@ -870,8 +870,10 @@ __global__ __launch_bounds__(256) void k_wfs_m(KARGS, int xsel) {
                     RT h[3];
 #pragma unroll
                     for (int k = 0; k < 3; k++) h[k] = (RT(1) - fx) * (RT)t[k * nxl] + fx * (RT)t[k * nxl + 1];
-                    v[0][si] += (RT(1) - fy) * h[0] + fy * h[1];
-                    v[1][si] += (RT(1) - fy) * h[1] + fy * h[2];
+                    // two fused multiply-adds a point, not a product, one
+                    // and an add: the FP64 issue is what bounds this pass
+                    v[0][si] = (RT(1) - fy) * h[0] + (fy * h[1] + v[0][si]);
+                    v[1][si] = (RT(1) - fy) * h[1] + (fy * h[2] + v[1][si]);
                 }
             } else {
 #pragma unroll
@@ -1034,7 +1036,8 @@ __global__ __launch_bounds__(256) void k_layer_m(KARGS, int psel_, int osel, int
                     if (si < ns) {
                         const RT *t = qw + si * qstride + o;
                         const RT q00 = t[0], q10 = t[1], q01 = t[G.pnx], q11 = t[G.pnx + 1];
-                        acc[si] += fy * ((RT(1) - fx) * q10 + fx * q00) + (RT(1) - fy) * ((RT(1) - fx) * q11 + fx * q01);
+                        acc[si] = fy * ((RT(1) - fx) * q10 + fx * q00) +
+                                  ((RT(1) - fy) * ((RT(1) - fx) * q11 + fx * q01) + acc[si]);
                     }
                 }
                 continue;
@@ -1202,8 +1205,8 @@ __global__ __launch_bounds__(128) void k_layer_m8(KARGS, int psel_, int osel, in
                 }
 #pragma unroll
                 for (int r = 0; r < R; r++) {
-                    acc[si][0][r] += fy * h0[r] + gy * h0[r + 1];
-                    acc[si][1][r] += fy * h1[r] + gy * h1[r + 1];
+                    acc[si][0][r] = fy * h0[r] + (gy * h0[r + 1] + acc[si][0][r]);
+                    acc[si][1][r] = fy * h1[r] + (gy * h1[r + 1] + acc[si][1][r]);
                 }
             }
         }

@@ -214,7 +214,7 @@ struct gpu_tomo {
     // systems per workgroup chosen by the autotuner (0: heuristic)
     int tune_wfs = 0, tune_layer = 0, tune_col = 0;
     long gen = 0;         // bumped whenever the launch tables must be rebuilt (shape, precision)
-    int tune_lty = 0;     // layer tile rows: 0 = heuristic (LTY where it fits), TILE or LTY
+    int tune_lty = 0;     // layer tile rows: 0 = built-in choice (default_lty), TILE, LTY2 or LTY
     int tune_colfft = 0;  // column kernel: 0 = registers where available, 1 = registers, 2 = LDS stages
     bool colr_ok = false; // the register column kernel applies (per-frequency blocks, ny = shL x shP)
     bool lty_ok = false;  // LTY-row tiles fit every layer of this (matched) plan
@@ -438,6 +438,20 @@ void build_mreg(gpu_tomo *g, const std::vector<float2> &hM, const std::vector<in
     g->grp_blk_host = hgb;
 }
 
+// Layer tile rows of a matched plan without a tuned choice, from its own sizes
+// (a plan computes the same bits in every call).  Layers above LTY rows:
+// LTY2 (k_layer of the 30 m system, 64 / 32 / 16 rows at one system per
+// workgroup: 1 system 9.7 8.1 7.4, 32: 19.8 17.7 30.9, 256: 90 89 200 us).
+// Smaller ones: TILE rows for few systems, LTY2 from about 160 000 nodes in
+// the plan on (16 / 32 rows; 20 m of 4 layers, 16 384 nodes: 1 system 6.4 7.0,
+// 16: 8.0 7.4, 64: 19.5 11.8, 256: 61 29; 10 m, 5184 nodes: 16: 5.9 6.3, 32:
+// 7.1 6.5, 64: 10.5 7.6, 256: 25.5 15.2 us).
+constexpr long LTY2_NODES = 160000;
+int default_lty(const gpu_tomo *g) {
+    if (g->lty_ok) return LTY2;
+    return g->lty2_ok && g->G.nxtot * g->nbatch >= LTY2_NODES ? LTY2 : TILE;
+}
+
 void build_plan(gpu_tomo *g, const mt_recon_t *R) {
     if (!R || R->npsr <= 0 || R->npsr > MAXL || R->nwfs <= 0) fail(MT_EINVAL, "invalid recon (npsr/nwfs)");
     if (R->pos != 1 && R->pos != 2) fail(MT_EINVAL, "tomo.pos must be 1 or 2");
@@ -615,16 +629,13 @@ void build_plan(gpu_tomo *g, const mt_recon_t *R) {
     G.lty = TILE;
     for (int l = 0; l < R->npsr; l++)
         if (R->xnx[l] < TILE + 2 || R->xny[l] < TILE + 2) matched = 0;
-    if (matched) {
-        G.lty = LTY;
-        for (int l = 0; l < R->npsr; l++)
-            if (R->xny[l] < LTY + 2) G.lty = TILE;
-    }
-    g->lty_ok = G.lty == LTY;
-    g->lty2_ok = matched != 0;
-    for (int l = 0; l < R->npsr; l++)
+    g->lty_ok = g->lty2_ok = matched != 0;
+    for (int l = 0; l < R->npsr; l++) {
+        if (R->xny[l] < LTY + 2) g->lty_ok = false;
         if (R->xny[l] < LTY2 + 2) g->lty2_ok = false;
+    }
     G.matched = matched;
+    if (matched) G.lty = default_lty(g);
     g->mray.upload(hm);
     G.mray = g->mray.p;
     g->hx_nx.upload(hnx);
@@ -919,8 +930,8 @@ void apply_lty(gpu_tomo *g) {
     if (!g->G.matched) return;
     const int lty = g->tune_lty == TILE   ? TILE
                     : g->tune_lty == LTY2 ? (g->lty2_ok ? LTY2 : TILE)
-                    : g->lty_ok           ? LTY
-                                          : TILE;
+                    : g->tune_lty == LTY  ? (g->lty_ok ? LTY : TILE)
+                                          : default_lty(g);
     if (lty == g->G.lty) return;
     g->G.lty = lty;
     g->SC.npart_layer = layer_tiles(g->G) * g->G.npsr;
@@ -1120,12 +1131,13 @@ void build_stage(Batch &B, Stage &out, KeyF key, GridF grid, SubF fill,
 }
 int ceil_div(int a, int b) { return (a + b - 1) / b; }
 // Systems per workgroup: the most of cmax, cmax/2, .., 1 that keeps >= thresh
-// workgroups in the launch; jw = (workgroups per system, systems) per job.
-int pick_cs(const std::vector<std::pair<long, int>> &jw, int cmax, int thresh) {
+// workgroups in the launch (thresh4 for 4 systems); jw = (workgroups per
+// system, systems) per job.
+int pick_cs(const std::vector<std::pair<long, int>> &jw, int cmax, int thresh, int thresh4) {
     for (int cs = cmax; cs > 1; cs >>= 1) {
         long tot = 0;
         for (auto &p : jw) tot += p.first * ceil_div(p.second, cs);
-        if (tot >= thresh) return cs;
+        if (tot >= (cs == 4 ? thresh4 : thresh)) return cs;
     }
     return 1;
 }
@@ -1221,8 +1233,12 @@ std::unique_ptr<Batch> make_batch(const std::vector<gpu_tomo *> &plans, const st
                     const int tuned = b.plan[js[0]]->tune_wfs;
                     sb.cs = !sb.matched ? 1
                             : tuned     ? std::min(tuned, sb.pos == 1 ? 4 : 2)
+                                        // k_wfs_m of the 30 m system (96 workgroups each), 1 / 2 / 4
+                                        // systems: 16: 11.5 10.6 12.3, 32: 18.2 15.3 16.1, 64: 32 25.6
+                                        // 25.4 us; of the 20 m one (36): 32: 8.5 8.5 9.6, 64: 12.6 10.7
+                                        // 12.0, 128: 20.3 17.4 16.8
                                         : pick_cs(jw_of(js, [&](int j) { return (long)ptiles(j) * G(j).nwfs; }),
-                                                  sb.pos == 1 ? 4 : 2, 512);
+                                                  sb.pos == 1 ? 4 : 2, 512, 1100);
                 });
     build_stage(b, b.layer,
                 [&](int j, std::vector<int> &k) {
@@ -1237,8 +1253,14 @@ std::unique_ptr<Batch> make_batch(const std::vector<gpu_tomo *> &plans, const st
                     const int tuned = b.plan[js[0]]->tune_layer;
                     sb.cs = !sb.matched ? 1
                             : tuned     ? tuned
-                                        : pick_cs(jw_of(js, [&](int j) { return (long)layer_tiles(G(j)) * G(j).npsr; }),
-                                                  4, 512);
+                            // k_layer_m8: one system, at every size measured (30 m, 16 x 32
+                            // tiles, 1 / 2 / 4 systems: 32: 17.7 18.6 23.5, 256: 89 91 98 us).
+                            // k_layer_m: two once that leaves 1024 workgroups (10 m of 4 layers:
+                            // 32: 7.1 8.0 10.3, 64: 10.5 9.4 11.8, 256: 25.5 20.8 20.5)
+                            : G(js[0]).lty != TILE
+                                ? 1
+                                : pick_cs(jw_of(js, [&](int j) { return (long)layer_tiles(G(j)) * G(j).npsr; }),
+                                          2, 1024, 1024);
                 });
     if (b.precond) {
         build_stage(b, b.row, [&](int j, std::vector<int> &k) { k = row_key(j); return true; },
@@ -1308,7 +1330,7 @@ std::unique_ptr<Batch> make_batch(const std::vector<gpu_tomo *> &plans, const st
                         const int tuned = b.plan[js[0]]->tune_col;
                         sb.cs = tuned ? std::min(tuned, 4)
                                       : pick_cs(jw_of(js, [&](int j) { return (long)G(j).ngroup; }),
-                                                b.spec64 ? 2 : 4, 384);
+                                                b.spec64 ? 2 : 4, 384, 384);
                         auto fits = [&](int c) {
                             for (int j : js)
                                 if (col_lds(G(j).maxcol, G(j).npsr, G(j).fny, b.spec64, c) > lmax) return false;
