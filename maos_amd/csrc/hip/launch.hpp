@@ -14,6 +14,7 @@ struct LaunchTab {
     const Job *jobs;   // device
     const WGI *wgi;    // device, nwg entries
     int nwg;
+    Job one;           // the job of a launch of one (pd null: read jobs)
 };
 
 void launch_ttr(const LaunchTab &t, hipStream_t st);

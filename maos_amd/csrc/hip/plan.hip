@@ -138,6 +138,7 @@ struct Batch {
     // a job table to launch with instead of `jobs` (same jobs, other device
     // records: gpu_tomo_solve_dev_noalloc's workspace); null normally
     const Job *jobs_over = nullptr;
+    bool switched = false;  // jobs are switched on and off between launches (the request loop)
 };
 }  // namespace
 
@@ -1393,7 +1394,11 @@ void drop_batches(gpu_tomo *g) {
     g->own.clear();
 }
 
-LaunchTab tab(const Batch &B, const Sub &s) { return LaunchTab{B.jobs_over ? B.jobs_over : B.jobs.p, s.wgi.p, s.nwg}; }
+LaunchTab tab(const Batch &B, const Sub &s) {
+    LaunchTab t{B.jobs_over ? B.jobs_over : B.jobs.p, s.wgi.p, s.nwg, Job{}};
+    if (!B.jobs_over && !B.switched && B.hjob.size() == 1) t.one = B.hjob[0];
+    return t;
+}
 
 // Operator A v -> Ap for all jobs (WFS pass + layer pass).
 void enqueue_L(Batch &B, int vsel, int partsel, Rec &rec) {
@@ -2802,6 +2807,7 @@ void flight_build_body(gpu_tomo_server *S, Flight &f) {
         }
     if (pl.empty()) return;
     f.B = make_batch(pl, std::vector<int>(pl.size(), 0), std::vector<int>(pl.size(), 1));
+    f.B->switched = true;
     HIPCHK(hipHostMalloc((void **)&f.hjobs, sizeof(Job) * pl.size()));
     f.hoff.resize(pl.size());
     f.nin = f.nout = f.nres = 0;
