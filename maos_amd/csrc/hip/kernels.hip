@@ -787,9 +787,18 @@ __global__ __launch_bounds__(256) void k_layer(KARGS, int psel_, int osel, int p
 // mirror.  Layer windows (k_wfs_m) and WFS-field windows (k_layer_m) are
 // staged in LDS with coalesced loads.
 // ---------------------------------------------------------------------------
-template <int POS, typename RT, int CS>
-__global__ __launch_bounds__(256) void k_wfs_m(KARGS, int xsel) {
+// Few systems leave the chip nearly empty and a workgroup waits for its chain
+// of layers (k_layer: WFS), a round trip to memory each.  With WS > 1 the
+// workgroup has WS groups of threads that take the layers (WFS) in turn; their
+// terms go to LDS and are added in the order of the loop, so the bits are
+// those of WS = 1.  One 30 m system: k_wfs_m 6.1 -> 5.3, k_layer_m8 7.6 -> 6.2 us.
+constexpr int WSMAX = 8;  // most layers (WFS) of the split forms
+template <int POS, typename RT, int CS, int WS = 1>
+__global__ __launch_bounds__(256 * WS) void k_wfs_m(KARGS, int xsel) {
     KJOB;
+    static_assert(WS == 1 || CS == 1, "the split form takes one system");
+    const int tid = WS > 1 ? (int)threadIdx.x & 255 : (int)threadIdx.x;
+    const int grp = WS > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8) : 0;
     const float *x = vsel(PD, xsel);
     RT *q = (RT *)PD.q;
     constexpr int H = TILE + 2 * POS;   // opd window edge
@@ -801,6 +810,7 @@ __global__ __launch_bounds__(256) void k_wfs_m(KARGS, int xsel) {
     __shared__ float2 gps[S2 * NP2];  // GP coefficients of the window's corners
     __shared__ RT opd[CS][H * H];
     __shared__ RT wgx[CS][S2], wgy[CS][S2];
+    __shared__ RT term[WS > 1 ? WSMAX * H * H : 1];  // [layer][2 rows][item]
     const int w = by, s0 = J.s0 + bz * CS, ns = min(CS, J.s0 + J.nsys - s0);
     const int pnx = G.pnx, pny = G.pny;
     const int ntx = (pnx + TILE - 1) / TILE;
@@ -815,7 +825,7 @@ __global__ __launch_bounds__(256) void k_wfs_m(KARGS, int xsel) {
     float4 nv[UN];
 #pragma unroll
     for (int u = 0; u < UG; u++) {
-        const int i = min((int)threadIdx.x + 256 * u, S2 * NP2 - 1);
+        const int i = min(tid + 256 * u, S2 * NP2 - 1);
         const int c = i / NP2, z = i - c * NP2;
         const int cx = tx0 - POS + c % S, cy = ty0 - POS + c / S;
         const int cxc = min(max(cx, 0), pnx - 1), cyc = min(max(cy, 0), pny - 1);
@@ -824,7 +834,7 @@ __global__ __launch_bounds__(256) void k_wfs_m(KARGS, int xsel) {
     }
 #pragma unroll
     for (int u = 0; u < UN; u++) {
-        const int i = threadIdx.x + 256 * u;
+        const int i = tid + 256 * u;
         const int ic = min(i, S2 - 1);
         const int cx = tx0 - POS + ic % S, cy = ty0 - POS + ic / S;
         const int cxc = min(max(cx, 0), pnx - 1), cyc = min(max(cy, 0), pny - 1);
@@ -834,7 +844,7 @@ __global__ __launch_bounds__(256) void k_wfs_m(KARGS, int xsel) {
 #pragma unroll
     for (int u = 0; u < UG; u++) {
         // past the end: the last entry again, with its own value
-        const int i = min((int)threadIdx.x + 256 * u, S2 * NP2 - 1);
+        const int i = min(tid + 256 * u, S2 * NP2 - 1);
         gps[i] = gv[u];
     }
     // HX on the opd window, gathered straight from the layers (L1/L2 hits):
@@ -846,8 +856,8 @@ __global__ __launch_bounds__(256) void k_wfs_m(KARGS, int xsel) {
     // Work item i: column i % H of the window, rows 2*(i / H) and +1 (H is
     // even), so on the plain path the middle sample row serves both points.
     constexpr int NI = H * H / 2;
-    const int ia = threadIdx.x % H, ib = threadIdx.x / H;
-    const bool item = threadIdx.x < NI;
+    const int ia = tid % H, ib = tid / H;
+    const bool item = tid < NI;
     const int hx = tx0 - POS + ia, hy0 = ty0 - POS + 2 * ib;
     RT v[2][CS];
 #pragma unroll
@@ -856,7 +866,7 @@ __global__ __launch_bounds__(256) void k_wfs_m(KARGS, int xsel) {
         for (int si = 0; si < CS; si++) v[r][si] = 0;
     if (item) {
         const float *xs = x + (long)s0 * G.nxtot;
-        for (int l = 0; l < G.npsr; l++) {
+        for (int l = grp; l < G.npsr; l += WS) {
             const MRay m = mray(G, w * MAXL + l);
             const int nxl = G.xnx[l], nyl = G.xny[l];
             const long xo = G.xoff[l];
@@ -876,10 +886,13 @@ __global__ __launch_bounds__(256) void k_wfs_m(KARGS, int xsel) {
                     RT h[3];
 #pragma unroll
                     for (int k = 0; k < 3; k++) h[k] = (RT(1) - fx) * (RT)t[k * nxl] + fx * (RT)t[k * nxl + 1];
-                    // two fused multiply-adds a point, not a product, one
-                    // and an add: the FP64 issue is what bounds this pass
-                    v[0][si] = (RT(1) - fy) * h[0] + (fy * h[1] + v[0][si]);
-                    v[1][si] = (RT(1) - fy) * h[1] + (fy * h[2] + v[1][si]);
+                    if constexpr (WS > 1) {
+                        v[0][si] = (RT(1) - fy) * h[0] + fy * h[1];
+                        v[1][si] = (RT(1) - fy) * h[1] + fy * h[2];
+                    } else {
+                        v[0][si] += (RT(1) - fy) * h[0] + fy * h[1];
+                        v[1][si] += (RT(1) - fy) * h[1] + fy * h[2];
+                    }
                 }
             } else {
 #pragma unroll
@@ -896,23 +909,37 @@ __global__ __launch_bounds__(256) void k_wfs_m(KARGS, int xsel) {
                         const float *t = xl + (long)min(si, ns - 1) * G.nxtot;
                         const RT a = t[o00], b = t[o10], c = t[o01], d = t[o11];
                         const RT h = (RT(1) - fy) * ((RT(1) - fx) * a + fx * b) + fy * ((RT(1) - fx) * c + fx * d);
-                        v[r][si] += ok ? h : RT(0);
+                        if constexpr (WS > 1) v[r][si] = ok ? h : RT(0);
+                        else v[r][si] += ok ? h : RT(0);
                     }
                 }
             }
+            if constexpr (WS > 1) {
+                term[(2 * l) * NI + tid] = v[0][0];
+                term[(2 * l + 1) * NI + tid] = v[1][0];
+            }
         }
+        if constexpr (WS == 1)
 #pragma unroll
-        for (int r = 0; r < 2; r++)
+            for (int r = 0; r < 2; r++)
 #pragma unroll
-            for (int si = 0; si < CS; si++)
-                if (si < ns) opd[si][(2 * ib + r) * H + ia] = v[r][si];
+                for (int si = 0; si < CS; si++)
+                    if (si < ns) opd[si][(2 * ib + r) * H + ia] = v[r][si];
+    }
+    if constexpr (WS > 1) {
+        __syncthreads();
+        if (grp < 2 && item) {  // group r adds row r of its items
+            RT a = 0;
+            for (int l = 0; l < G.npsr; l++) a += term[(2 * l + grp) * NI + tid];
+            opd[0][(2 * ib + grp) * H + ia] = a;
+        }
     }
     __syncthreads();
     // W GP per subaperture corner of the window (zero coefficients where none)
 #pragma unroll
     for (int u = 0; u < UN; u++) {
-        const int i = threadIdx.x + 256 * u;
-        if (i < S2) {
+        const int i = tid + 256 * u;
+        if (i < S2 && grp == 0) {
             const int a = i % S, b = i / S;
             float2 c[NP2];
 #pragma unroll
@@ -938,9 +965,9 @@ __global__ __launch_bounds__(256) void k_wfs_m(KARGS, int xsel) {
     }
     __syncthreads();
     // GP' gather onto the tile
-    const int ox = threadIdx.x % TILE, oy = threadIdx.x / TILE;
+    const int ox = tid % TILE, oy = tid / TILE;
     const int px = tx0 + ox, py = ty0 + oy;
-    if (threadIdx.x < TILE * TILE && px < pnx && py < pny) {
+    if (grp == 0 && tid < TILE * TILE && px < pnx && py < pny) {
         float2 c[NP2];
         int sidx[NP2];
 #pragma unroll
@@ -963,9 +990,13 @@ __global__ __launch_bounds__(256) void k_wfs_m(KARGS, int xsel) {
     }
 }
 
-template <bool LHS, typename RT, int CS>
-__global__ __launch_bounds__(256) void k_layer_m(KARGS, int psel_, int osel, int partsel) {
+template <bool LHS, typename RT, int CS, int WS = 1>
+__global__ __launch_bounds__(256 * WS) void k_layer_m(KARGS, int psel_, int osel, int partsel) {
     KJOB;
+    static_assert(WS == 1 || CS == 1, "the split form takes one system");
+    const int tid = WS > 1 ? (int)threadIdx.x & 255 : (int)threadIdx.x;
+    const int grp = WS > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8) : 0;
+    __shared__ RT term[WS > 1 ? WSMAX * 256 : 1];  // [WFS][node]
     const RT *q = (const RT *)PD.q;
     const float *p = vsel(PD, psel_);
     RT *out = rsel<RT>(PD, osel);
@@ -975,20 +1006,20 @@ __global__ __launch_bounds__(256) void k_layer_m(KARGS, int psel_, int osel, int
     constexpr int PH2 = PH * PH;
     constexpr int UP = (PH2 + 255) / 256;
     __shared__ float ps[CS][LHS ? PH2 : 1];
-    __shared__ double sh[8];
+    __shared__ double sh[4 * WS + 4];
     const int l = by, s0 = J.s0 + bz * CS, ns = min(CS, J.s0 + J.nsys - s0);
     const int nxl = G.xnx[l], nyl = G.xny[l];
     const int ntx = (nxl + TILE - 1) / TILE, nty = (nyl + TILE - 1) / TILE;
     const bool active = bx < ntx * nty;
     const int jx0 = (bx % ntx) * TILE, jy0 = (bx / ntx) * TILE;
-    const int jx = jx0 + (int)threadIdx.x % TILE, jy = jy0 + (int)threadIdx.x / TILE;
+    const int jx = jx0 + tid % TILE, jy = jy0 + tid / TILE;
     const bool mine = active && jx < nxl && jy < nyl;
-    if (LHS && active) {
+    if (LHS && active && grp == 0) {
         // p windows, periodic (layers are >= TILE + 2, so one wrap suffices)
         int off[UP];
 #pragma unroll
         for (int u = 0; u < UP; u++) {
-            const int i = threadIdx.x + 256 * u;
+            const int i = tid + 256 * u;
             int xx = jx0 - 2 + i % PH, yy = jy0 - 2 + i / PH;
             xx += xx < 0 ? nxl : 0;
             xx -= xx >= nxl ? nxl : 0;
@@ -1002,7 +1033,7 @@ __global__ __launch_bounds__(256) void k_layer_m(KARGS, int psel_, int osel, int
             const float *pl = p + (long)(s0 + si) * G.nxtot + G.xoff[l];
 #pragma unroll
             for (int u = 0; u < UP; u++) {
-                const int i = threadIdx.x + 256 * u;
+                const int i = tid + 256 * u;
                 pv[si][u] = (si < ns && i < PH2) ? pl[off[u]] : 0.f;
             }
         }
@@ -1010,7 +1041,7 @@ __global__ __launch_bounds__(256) void k_layer_m(KARGS, int psel_, int osel, int
         for (int si = 0; si < CS; si++)
 #pragma unroll
             for (int u = 0; u < UP; u++) {
-                const int i = threadIdx.x + 256 * u;
+                const int i = tid + 256 * u;
                 if (i < PH2) ps[si][i] = pv[si][u];
             }
     }
@@ -1026,8 +1057,9 @@ __global__ __launch_bounds__(256) void k_layer_m(KARGS, int psel_, int osel, int
     for (int si = 0; si < CS; si++) acc[si] = 0;
     const int tw = min(TILE, nxl - jx0), th = min(TILE, nyl - jy0);
     if (mine) {
-        for (int w = 0; w < G.nwfs; w++) {
+        for (int w = grp; w < G.nwfs; w += WS) {
             const MRay m = mray(G, w * MAXL + l);
+            if constexpr (WS > 1) term[w * 256 + tid] = 0;
             const bool edgex = m.wx && jx0 == 0, edgey = m.wy && jy0 == 0;
             if (!edgex && (jx0 + tw - 1 - m.cx < m.ax0 || jx0 - m.cx - 1 >= m.ax1)) continue;
             if (!edgey && (jy0 + th - 1 - m.cy < m.ay0 || jy0 - m.cy - 1 >= m.ay1)) continue;
@@ -1042,8 +1074,9 @@ __global__ __launch_bounds__(256) void k_layer_m(KARGS, int psel_, int osel, int
                     if (si < ns) {
                         const RT *t = qw + si * qstride + o;
                         const RT q00 = t[0], q10 = t[1], q01 = t[G.pnx], q11 = t[G.pnx + 1];
-                        acc[si] = fy * ((RT(1) - fx) * q10 + fx * q00) +
-                                  ((RT(1) - fy) * ((RT(1) - fx) * q11 + fx * q01) + acc[si]);
+                        const RT c = fy * ((RT(1) - fx) * q10 + fx * q00) + (RT(1) - fy) * ((RT(1) - fx) * q11 + fx * q01);
+                        if constexpr (WS > 1) term[w * 256 + tid] = c;
+                        else acc[si] += c;
                     }
                 }
                 continue;
@@ -1065,20 +1098,26 @@ __global__ __launch_bounds__(256) void k_layer_m(KARGS, int psel_, int osel, int
             for (int si = 0; si < CS; si++) {
                 if (si < ns) {
                     const RT *t = qw + si * qstride;
-                    acc[si] += wy0 * (wx1 * t[o10] + wx0 * t[o00]) + wy1 * (wx1 * t[o11] + wx0 * t[o01]);
+                    const RT c = wy0 * (wx1 * t[o10] + wx0 * t[o00]) + wy1 * (wx1 * t[o11] + wx0 * t[o01]);
+                    if constexpr (WS > 1) term[w * 256 + tid] = c;
+                    else acc[si] += c;
                 }
             }
         }
     }
-    if (LHS) __syncthreads();
+    if (LHS || WS > 1) __syncthreads();
+    if constexpr (WS > 1) {
+        if (grp == 0 && mine)
+            for (int w = 0; w < G.nwfs; w++) acc[0] += term[w * 256 + tid];
+    }
     double dot[CS];
 #pragma unroll
     for (int si = 0; si < CS; si++) {
         dot[si] = 0;
-        if (mine && si < ns) {
+        if (mine && si < ns && grp == 0) {
             RT a = acc[si];
             if (LHS) {
-                const int tx = threadIdx.x % TILE, ty = threadIdx.x / TILE;
+                const int tx = tid % TILE, ty = tid / TILE;
                 const float *P0 = ps[si] + (ty + 2) * PH + tx + 2;
                 auto P = [&](int dx, int dy) { return (RT)P0[dy * PH + dx]; };
                 const RT c = P(0, 0);
@@ -1108,25 +1147,29 @@ __global__ __launch_bounds__(256) void k_layer_m(KARGS, int psel_, int osel, int
 // k_layer_m (the reference's bilinear transpose):
 //   acc += fy (gx q[iy0, ix1] + fx q[iy0, ix0]) + gy (gx q[iy1, ix1] + fx q[iy1, ix0]),
 // gx = 1 - fx, gy = 1 - fy; the p.Ap partial of a thread sums its nodes.
-template <bool LHS, typename RT, int CS, int LT>
-__global__ __launch_bounds__(128) void k_layer_m8(KARGS, int psel_, int osel, int partsel) {
+template <bool LHS, typename RT, int CS, int LT, int WS = 1>
+__global__ __launch_bounds__(128 * WS) void k_layer_m8(KARGS, int psel_, int osel, int partsel) {
     KJOB;
+    static_assert(WS == 1 || CS == 1, "the split form takes one system");
+    const int tid = WS > 1 ? (int)threadIdx.x & 127 : (int)threadIdx.x;
+    const int grp = WS > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 7) : 0;
     const RT *q = (const RT *)PD.q;
     const float *p = vsel(PD, psel_);
     RT *out = rsel<RT>(PD, osel);
     double *part = psel(PD, partsel);
     const int partstride = PD.SC.maxpart;
-    constexpr int R = LT / 16, NT = 128;
+    constexpr int R = LT / 16, NT = 128 * WS;
     constexpr int PW = TILE + 4, PHH = LT + 4, P2 = PW * PHH;  // p window (L2'L2 reach 2)
     constexpr int UP = (P2 + NT - 1) / NT;
     __shared__ float ps[CS][LHS ? P2 : 1];
-    __shared__ double sh[8];
+    __shared__ double sh[2 * WS + 6];
+    __shared__ RT term[WS > 1 ? WSMAX * 2 * R * 128 : 1];  // [WFS][node of the thread][thread]
     const int l = by, s0 = J.s0 + bz * CS, ns = min(CS, J.s0 + J.nsys - s0);
     const int nxl = G.xnx[l], nyl = G.xny[l];
     const int ntx = (nxl + TILE - 1) / TILE, nty = (nyl + LT - 1) / LT;
     const bool active = bx < ntx * nty;
     const int jx0 = (bx % ntx) * TILE, jy0 = (bx / ntx) * LT;
-    const int tx = threadIdx.x % (TILE / 2), ty = threadIdx.x / (TILE / 2);
+    const int tx = tid % (TILE / 2), ty = tid / (TILE / 2);
     const int jx = jx0 + 2 * tx, jyb = jy0 + R * ty;
     const int nr = active ? max(0, min(R, nyl - jyb)) : 0;  // rows of this thread
     const int nc = active ? max(0, min(2, nxl - jx)) : 0;   // columns of this thread
@@ -1176,14 +1219,20 @@ __global__ __launch_bounds__(128) void k_layer_m8(KARGS, int psel_, int osel, in
         const RT *qs[CS];  // the WFS fields of each system
 #pragma unroll
         for (int si = 0; si < CS; si++) qs[si] = q + (long)(s0 + min(si, ns - 1)) * G.nwfs * G.nploc;
-        for (int w = 0; w < G.nwfs; w++) {
+        for (int w = grp; w < G.nwfs; w += WS) {
             const MRay m = mray(G, w * MAXL + l);
+            RT *tm = term + w * (2 * R * 128) + tid;
             // the whole record in one scalar round trip (the compiler would
             // otherwise load the fields used after the tile test separately)
             asm volatile("" ::"s"(m.fx), "s"(m.fy), "s"(m.nrow), "s"(m.qoff));
             const bool edgex = m.wx && jx0 == 0, edgey = m.wy && jy0 == 0;
-            if (!edgex && (jx0 + tw - 1 - m.cx < m.ax0 || jx0 - m.cx - 1 >= m.ax1)) continue;
-            if (!edgey && (jy0 + th - 1 - m.cy < m.ay0 || jy0 - m.cy - 1 >= m.ay1)) continue;
+            if ((!edgex && (jx0 + tw - 1 - m.cx < m.ax0 || jx0 - m.cx - 1 >= m.ax1)) ||
+                (!edgey && (jy0 + th - 1 - m.cy < m.ay0 || jy0 - m.cy - 1 >= m.ay1))) {
+                if constexpr (WS > 1)
+#pragma unroll
+                    for (int c = 0; c < 2 * R; c++) tm[c * 128] = 0;
+                continue;
+            }
             const RT fx = m.fx, fy = m.fy, gx = RT(1) - fx, gy = RT(1) - fy;
             const int ixa = (m.wx && jx == 0) ? m.ax1 - 1 : jx - m.cx - 1, ixb = jx - m.cx, ixc = ixb + 1;
             const bool va = ixa >= m.ax0 && ixa < m.ax1, vb = ixb >= m.ax0 && ixb < m.ax1,
@@ -1211,18 +1260,32 @@ __global__ __launch_bounds__(128) void k_layer_m8(KARGS, int psel_, int osel, in
                 }
 #pragma unroll
                 for (int r = 0; r < R; r++) {
-                    acc[si][0][r] = fy * h0[r] + (gy * h0[r + 1] + acc[si][0][r]);
-                    acc[si][1][r] = fy * h1[r] + (gy * h1[r + 1] + acc[si][1][r]);
+                    const RT c0 = fy * h0[r] + gy * h0[r + 1], c1 = fy * h1[r] + gy * h1[r + 1];
+                    if constexpr (WS > 1) {
+                        tm[r * 128] = c0;
+                        tm[(R + r) * 128] = c1;
+                    } else {
+                        acc[si][0][r] += c0;
+                        acc[si][1][r] += c1;
+                    }
                 }
             }
         }
     }
-    if (LHS) __syncthreads();
+    if (LHS || WS > 1) __syncthreads();
+    if constexpr (WS > 1) {
+        if (grp == 0 && nr > 0 && nc > 0)
+            for (int w = 0; w < G.nwfs; w++)
+#pragma unroll
+                for (int c = 0; c < 2; c++)
+#pragma unroll
+                    for (int r = 0; r < R; r++) acc[0][c][r] += term[w * (2 * R * 128) + (c * R + r) * 128 + tid];
+    }
     double dot[CS];
 #pragma unroll
     for (int si = 0; si < CS; si++) {
         dot[si] = 0;
-        if (si < ns) {
+        if (si < ns && grp == 0) {
 #pragma unroll
             for (int c = 0; c < 2; c++) {
                 if (c >= nc) continue;
@@ -1552,6 +1615,10 @@ __global__ __launch_bounds__(256) void k_col(KARGS) {
     const int nrow = (b1 - b0) * bs;
     constexpr int RP = BS > 0 ? 3 : 1;
     constexpr int BR = BS > 0 ? BS : 1;
+    // (the column offsets first: their loads are waited for before the block
+    // rows' are, which a scalar loop over the columns would each be alone)
+    const int ic = min((int)threadIdx.x, ncg * npsr - 1), icc = fdiv(ic, ldf(G.dnpsr));
+    const int cof = (int)G.soff[ic - icc * npsr] + G.colkx[c0 + icc] * ny;
     float2 mr[RP][BR];
     int pr[RP][BR], pmr[RP];
     if constexpr (BS > 0) {
@@ -1570,12 +1637,10 @@ __global__ __launch_bounds__(256) void k_col(KARGS) {
             pmr[u] = bp[m];
         }
     }
-    // (uniform loop: scalar loads, which do not wait behind the vector loads
-    // above)
-    for (int ci = 0; ci < ncg; ci++) {
-        const int kx = ((const CONSTAS int *)G.colkx)[c0 + ci];
-        for (int l = 0; l < npsr; l++)
-            if (threadIdx.x == 0) coff[ci * npsr + l] = (int)G.soff[l] + kx * ny;
+    if ((int)threadIdx.x < ncg * npsr) coff[threadIdx.x] = cof;
+    for (int i = threadIdx.x + 256; i < ncg * npsr; i += 256) {
+        const int ci = fdiv(i, ldf(G.dnpsr));
+        coff[i] = (int)G.soff[i - ci * npsr] + G.colkx[c0 + ci] * ny;
     }
     __syncthreads();
     // Twiddles and spectrum columns: U loads in flight per thread,
@@ -2123,7 +2188,8 @@ static void launch_wfs_rt(const LaunchTab &t, bool rhs, int matched, int pos, in
         if (pos == 1) hipLaunchKernelGGL((k_wfs<1, false, RT>), grid, blk, 0, st, KT, xsel);
         else hipLaunchKernelGGL((k_wfs<2, false, RT>), grid, blk, 0, st, KT, xsel);
     } else if (pos == 1) {
-        if (cs == 4) hipLaunchKernelGGL((k_wfs_m<1, RT, 4>), grid, blk, 0, st, KT, xsel);
+        if (cs < 0) hipLaunchKernelGGL((k_wfs_m<1, RT, 1, 4>), grid, dim3(1024), 0, st, KT, xsel);
+        else if (cs == 4) hipLaunchKernelGGL((k_wfs_m<1, RT, 4>), grid, blk, 0, st, KT, xsel);
         else if (cs == 2) hipLaunchKernelGGL((k_wfs_m<1, RT, 2>), grid, blk, 0, st, KT, xsel);
         else hipLaunchKernelGGL((k_wfs_m<1, RT, 1>), grid, blk, 0, st, KT, xsel);
     } else {
@@ -2147,10 +2213,12 @@ static void launch_layer_rt(const LaunchTab &t, int matched, int cs, int psel_, 
         else hipLaunchKernelGGL((k_layer_m8<LHS, RT, 1, LTY>), grid, b8, 0, st, KT, psel_, osel, partsel);
     } else if (matched == 3) {  // 16 x 32 tiles
         const dim3 b8(128);
-        if (cs == 4) hipLaunchKernelGGL((k_layer_m8<LHS, RT, 4, LTY2>), grid, b8, 0, st, KT, psel_, osel, partsel);
+        if (cs < 0) hipLaunchKernelGGL((k_layer_m8<LHS, RT, 1, LTY2, 6>), grid, dim3(768), 0, st, KT, psel_, osel, partsel);
+        else if (cs == 4) hipLaunchKernelGGL((k_layer_m8<LHS, RT, 4, LTY2>), grid, b8, 0, st, KT, psel_, osel, partsel);
         else if (cs == 2) hipLaunchKernelGGL((k_layer_m8<LHS, RT, 2, LTY2>), grid, b8, 0, st, KT, psel_, osel, partsel);
         else hipLaunchKernelGGL((k_layer_m8<LHS, RT, 1, LTY2>), grid, b8, 0, st, KT, psel_, osel, partsel);
     }
+    else if (cs < 0) hipLaunchKernelGGL((k_layer_m<LHS, RT, 1, 4>), grid, dim3(1024), 0, st, KT, psel_, osel, partsel);
     else if (cs == 4) hipLaunchKernelGGL((k_layer_m<LHS, RT, 4>), grid, blk, 0, st, KT, psel_, osel, partsel);
     else if (cs == 2) hipLaunchKernelGGL((k_layer_m<LHS, RT, 2>), grid, blk, 0, st, KT, psel_, osel, partsel);
     else hipLaunchKernelGGL((k_layer_m<LHS, RT, 1>), grid, blk, 0, st, KT, psel_, osel, partsel);
@@ -2266,6 +2334,12 @@ static void launch_colr_t(const LaunchTab &t, int P, int L, int bs, int nthr, si
     if (L == 32 && P == 3 && bs == 6) hipLaunchKernelGGL((k_colr<FT, 3, 32, 6>), grid, blk, lds, st, KT);
     else if (L == 32 && P == 3) hipLaunchKernelGGL((k_colr<FT, 3, 32, 0>), grid, blk, lds, st, KT);
     else if (L == 32 && P == 2) hipLaunchKernelGGL((k_colr<FT, 2, 32, 0>), grid, blk, lds, st, KT);
+    // columns of 28, 56, 40, 80 and 48 points
+    else if (L == 4 && P == 7) hipLaunchKernelGGL((k_colr<FT, 7, 4, 0>), grid, blk, lds, st, KT);
+    else if (L == 8 && P == 7) hipLaunchKernelGGL((k_colr<FT, 7, 8, 0>), grid, blk, lds, st, KT);
+    else if (L == 8 && P == 5) hipLaunchKernelGGL((k_colr<FT, 5, 8, 0>), grid, blk, lds, st, KT);
+    else if (L == 16 && P == 5) hipLaunchKernelGGL((k_colr<FT, 5, 16, 0>), grid, blk, lds, st, KT);
+    else if (L == 16 && P == 3) hipLaunchKernelGGL((k_colr<FT, 3, 16, 0>), grid, blk, lds, st, KT);
     else switch (P) {
         case 2: hipLaunchKernelGGL((k_colr<FT, 2, 0, 0>), grid, blk, lds, st, KT); break;
         case 3: hipLaunchKernelGGL((k_colr<FT, 3, 0, 0>), grid, blk, lds, st, KT); break;

@@ -19,6 +19,9 @@ struct LaunchTab {
 
 void launch_ttr(const LaunchTab &t, hipStream_t st);
 // rt64: the residual-side arrays (q, Ap, b, r) are double instead of float.
+// cs: systems per workgroup of the matched kernels; negative: one, in the
+// split form (few workgroups; at most 8 layers and WFS, and layer tiles of
+// TILE or LTY2 rows).
 void launch_wfs(const LaunchTab &t, bool rhs, int matched, int pos, int cs, int rt64, int xsel, hipStream_t st);
 void launch_layer(const LaunchTab &t, bool lhs, int matched, int cs, int rt64, int psel, int osel, int partsel,
                   hipStream_t st);

@@ -120,6 +120,7 @@ struct Sub {
     int rp = 0;   // row stages: P of the register row FFT (rows of 32 P points), or 0
     int nthr = 0; // its threads per workgroup
     int regL = 0; // its lanes per column FFT (shL of every job)
+    bool split = false;  // WFS and layer stages: the split form
     size_t lds = 0;
     DevBuf<WGI> wgi;
     int nwg = 0;
@@ -1143,6 +1144,14 @@ int pick_cs(const std::vector<std::pair<long, int>> &jw, int cmax, int thresh, i
     return 1;
 }
 
+// Launches of at most this many workgroups (one per CU) take the split forms
+// of k_wfs_m (tomo.pos = 1) and the layer kernels.  us per launch, back to back,
+// whole / split: k_layer_m8 of the 30 m system (108 workgroups each) 1 system
+// 7.6 6.2, 2: 7.6 6.2, 4: 7.8 10.3; k_layer_m of the 20 m one (64) 4: 5.8 5.2, 6:
+// 5.9 6.8; k_wfs_m of the 30 m one (96) 1: 6.1 5.3, 4: 6.7 7.6, of the 20 m one
+// (36) 4: 5.1 5.0, 8: 5.4 6.7; with tomo.pos = 2 (ngs8) 1: 5.1 6.0.
+constexpr long SPLIT_WGS = 256;
+
 std::unique_ptr<Batch> make_batch(const std::vector<gpu_tomo *> &plans, const std::vector<int> &s0,
                                   const std::vector<int> &nsys) {
     std::unique_ptr<Batch> B(new Batch());
@@ -1172,6 +1181,16 @@ std::unique_ptr<Batch> make_batch(const std::vector<gpu_tomo *> &plans, const st
         std::vector<std::pair<long, int>> v;
         for (int j : js) v.push_back({per(j), NS(j)});
         return v;
+    };
+    auto wgs = [&](const std::vector<int> &js, std::function<long(int)> per) {
+        long tot = 0;
+        for (int j : js) tot += per(j) * NS(j);
+        return tot;
+    };
+    auto can_split = [&](const std::vector<int> &js) {
+        for (int j : js)
+            if (G(j).npsr > 8 || G(j).nwfs > 8) return false;
+        return true;
     };
     // A batch over several plans (uneven groups, the request loop) is mostly
     // small systems, whose kernels are short enough that the number of
@@ -1240,6 +1259,8 @@ std::unique_ptr<Batch> make_batch(const std::vector<gpu_tomo *> &plans, const st
                                         // 12.0, 128: 20.3 17.4 16.8
                                         : pick_cs(jw_of(js, [&](int j) { return (long)ptiles(j) * G(j).nwfs; }),
                                                   sb.pos == 1 ? 4 : 2, 512, 1100);
+                    sb.split = sb.matched && sb.pos == 1 && sb.cs == 1 && can_split(js) &&
+                               wgs(js, [&](int j) { return (long)ptiles(j) * G(j).nwfs; }) <= SPLIT_WGS;
                 });
     build_stage(b, b.layer,
                 [&](int j, std::vector<int> &k) {
@@ -1262,6 +1283,8 @@ std::unique_ptr<Batch> make_batch(const std::vector<gpu_tomo *> &plans, const st
                                 ? 1
                                 : pick_cs(jw_of(js, [&](int j) { return (long)layer_tiles(G(j)) * G(j).npsr; }),
                                           2, 1024, 1024);
+                    sb.split = sb.matched && sb.cs == 1 && can_split(js) && G(js[0]).lty != LTY &&
+                               wgs(js, [&](int j) { return (long)layer_tiles(G(j)) * G(j).npsr; }) <= SPLIT_WGS;
                 });
     if (b.precond) {
         build_stage(b, b.row, [&](int j, std::vector<int> &k) { k = row_key(j); return true; },
@@ -1286,10 +1309,13 @@ std::unique_ptr<Batch> make_batch(const std::vector<gpu_tomo *> &plans, const st
         // same order, so the same bits) with the largest workgroup.
         auto colreg = [&](int j) { return b.plan[j]->colr_ok && b.plan[j]->tune_colfft != 2 ? G(j).shP : 0; };
         std::map<int, int> nthr_of_p;  // merged: largest workgroup per P
+        std::map<int, int> lanes_of_p;  // ... and its lanes, 0 where they differ
         for (size_t j = 0; j < b.hjob.size(); j++)
             if (colreg((int)j)) {
                 int &v = nthr_of_p[colreg((int)j)];
                 v = std::max(v, colr_shape(G((int)j).bs, G((int)j).shL, nullptr));
+                const auto it = lanes_of_p.emplace(colreg((int)j), G((int)j).shL).first;
+                if (it->second != G((int)j).shL) it->second = 0;
             }
         auto colr_tasks_of = [&](int j) {
             int T = 1;
@@ -1299,7 +1325,7 @@ std::unique_ptr<Batch> make_batch(const std::vector<gpu_tomo *> &plans, const st
         build_stage(b, b.col,
                     [&](int j, std::vector<int> &k) {
                         if (colreg(j)) {
-                            if (merge) k = {-1, colreg(j), nthr_of_p[colreg(j)], 0, 0};
+                            if (merge) k = {-1, colreg(j), nthr_of_p[colreg(j)], lanes_of_p[colreg(j)], 0};
                             else k = {-1, colreg(j), colr_shape(G(j).bs, G(j).shL, nullptr), G(j).shL, G(j).bs};
                             return true;
                         }
@@ -1403,14 +1429,14 @@ LaunchTab tab(const Batch &B, const Sub &s) {
 // Operator A v -> Ap for all jobs (WFS pass + layer pass).
 void enqueue_L(Batch &B, int vsel, int partsel, Rec &rec) {
     rec(KC_WFS, [&] {
-        for (auto &s : B.wfs_l) launch_wfs(tab(B, *s), false, s->matched, s->pos, s->cs, B.rt64, vsel, rec.st);
+        for (auto &s : B.wfs_l) launch_wfs(tab(B, *s), false, s->matched, s->pos, s->split ? -1 : s->cs, B.rt64, vsel, rec.st);
         // the two stages hold the same partitions (keyed by tomo.pos) in order
         for (size_t i = 0; i < B.wfs_g.size(); i++)
             launch_wfs_lhs_tt(tab(B, *B.wfs_g[i]), tab(B, *B.ttl[i]), B.wfs_g[i]->pos, B.rt64, vsel, rec.st);
     });
     rec(KC_LAYER, [&] {
         for (auto &s : B.layer)
-            launch_layer(tab(B, *s), true, s->matched, s->cs, B.rt64, vsel, BUF_AP, partsel, rec.st);
+            launch_layer(tab(B, *s), true, s->matched, s->split ? -1 : s->cs, B.rt64, vsel, BUF_AP, partsel, rec.st);
     });
 }
 // RHS b = HX' GP' W (I - TT PTT) g for all jobs.
@@ -1422,7 +1448,8 @@ void enqueue_R(Batch &B, Rec &rec) {
         for (auto &s : B.wfs_r) launch_wfs(tab(B, *s), true, 0, s->pos, 1, B.rt64, BUF_X, rec.st);
     });
     rec(KC_LAYER_RHS, [&] {
-        for (auto &s : B.layer) launch_layer(tab(B, *s), false, s->matched, s->cs, B.rt64, BUF_X, BUF_B, PART_BB, rec.st);
+        for (auto &s : B.layer)
+            launch_layer(tab(B, *s), false, s->matched, s->split ? -1 : s->cs, B.rt64, BUF_X, BUF_B, PART_BB, rec.st);
     });
 }
 void enqueue_row(Batch &B, int kc, int mode, int iter, int xsel, Rec &rec) {
