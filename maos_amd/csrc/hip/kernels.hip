@@ -175,9 +175,15 @@ __device__ double reduce_partials(const double *part, int n, double *sh, int f32
 __device__ __forceinline__ double dmul(double a, double b, int f32) {
     return f32 ? (double)((float)a * (float)b) : a * b;
 }
+__device__ __forceinline__ double dadd(double a, double b, int f32) {
+    return f32 ? (double)((float)a + (float)b) : a + b;
+}
 __device__ __forceinline__ double dfma(double a, double b, double c, int f32) {
     return f32 ? (double)fmaf((float)a, (float)b, (float)c) : a * b + c;
 }
+// wa a + wb b with the rounding fixed (the compiler picks which product to fuse
+// from its surroundings): the layer kernels agree bit for bit.
+template <typename T> __device__ __forceinline__ T lerp2(T wa, T a, T wb, T b) { return fma(wa, a, wb * b); }
 __device__ __forceinline__ double ddiv(double a, double b, int f32) {
     return f32 ? (double)((float)a / (float)b) : a / b;
 }
@@ -1074,7 +1080,8 @@ __global__ __launch_bounds__(256 * WS) void k_layer_m(KARGS, int psel_, int osel
                     if (si < ns) {
                         const RT *t = qw + si * qstride + o;
                         const RT q00 = t[0], q10 = t[1], q01 = t[G.pnx], q11 = t[G.pnx + 1];
-                        const RT c = fy * ((RT(1) - fx) * q10 + fx * q00) + (RT(1) - fy) * ((RT(1) - fx) * q11 + fx * q01);
+                        const RT gx = RT(1) - fx, gy = RT(1) - fy;
+                        const RT c = lerp2(fy, lerp2(fx, q00, gx, q10), gy, lerp2(fx, q01, gx, q11));
                         if constexpr (WS > 1) term[w * 256 + tid] = c;
                         else acc[si] += c;
                     }
@@ -1098,7 +1105,7 @@ __global__ __launch_bounds__(256 * WS) void k_layer_m(KARGS, int psel_, int osel
             for (int si = 0; si < CS; si++) {
                 if (si < ns) {
                     const RT *t = qw + si * qstride;
-                    const RT c = wy0 * (wx1 * t[o10] + wx0 * t[o00]) + wy1 * (wx1 * t[o11] + wx0 * t[o01]);
+                    const RT c = lerp2(wy0, lerp2(wx0, t[o00], wx1, t[o10]), wy1, lerp2(wx0, t[o01], wx1, t[o11]));
                     if constexpr (WS > 1) term[w * 256 + tid] = c;
                     else acc[si] += c;
                 }
@@ -1110,6 +1117,7 @@ __global__ __launch_bounds__(256 * WS) void k_layer_m(KARGS, int psel_, int osel
         if (grp == 0 && mine)
             for (int w = 0; w < G.nwfs; w++) acc[0] += term[w * 256 + tid];
     }
+    // p.Ap (b.b) of the tile, in the order of the layer tile sums (k_layer_m8)
     double dot[CS];
 #pragma unroll
     for (int si = 0; si < CS; si++) {
@@ -1134,9 +1142,14 @@ __global__ __launch_bounds__(256 * WS) void k_layer_m(KARGS, int psel_, int osel
     }
 #pragma unroll
     for (int si = 0; si < CS; si++) {
-        const double d = block_sum(dot[si], sh, G.dot32);
+        double d = dot[si];
+        for (int o : {1, 16, 32, 2, 4, 8}) d = dadd(d, __shfl_xor(d, o, 64), G.dot32);
+        if (si) __syncthreads();  // the previous system's strips are read
+        if ((threadIdx.x & 63) == 0 && grp == 0) sh[tid >> 6] = d;
+        __syncthreads();
         if (threadIdx.x == 0 && part && si < ns)
-            part[(long)(s0 + si) * partstride + by * PD.ltiles + bx] = d;
+            part[(long)(s0 + si) * partstride + by * PD.ltiles + bx] =
+                dadd(dadd(dadd(sh[0], sh[1], G.dot32), sh[2], G.dot32), sh[3], G.dot32);
     }
 }
 
@@ -1146,7 +1159,13 @@ __global__ __launch_bounds__(256 * WS) void k_layer_m(KARGS, int psel_, int osel
 // columns (the middle one serves both columns), feed 2 R nodes.  Same arithmetic per node as
 // k_layer_m (the reference's bilinear transpose):
 //   acc += fy (gx q[iy0, ix1] + fx q[iy0, ix0]) + gy (gx q[iy1, ix1] + fx q[iy1, ix0]),
-// gx = 1 - fx, gy = 1 - fy; the p.Ap partial of a thread sums its nodes.
+// gx = 1 - fx, gy = 1 - fy, and the same p.Ap partials, one per 16 x 16 nodes.
+//
+// Layer tile sums: the order is the same whatever kernel takes the tile, so
+// that the tile shape, chosen by the number of systems, does not change a bit.
+// A 16 x 16 tile is four strips of 4 rows, added in order.  In a strip, two
+// adjacent columns are added first, then two adjacent rows, then these pairs of
+// rows (a thread's nodes here), then the 8 column pairs as a tree.
 template <bool LHS, typename RT, int CS, int LT, int WS = 1>
 __global__ __launch_bounds__(128 * WS) void k_layer_m8(KARGS, int psel_, int osel, int partsel) {
     KJOB;
@@ -1162,7 +1181,6 @@ __global__ __launch_bounds__(128 * WS) void k_layer_m8(KARGS, int psel_, int ose
     constexpr int PW = TILE + 4, PHH = LT + 4, P2 = PW * PHH;  // p window (L2'L2 reach 2)
     constexpr int UP = (P2 + NT - 1) / NT;
     __shared__ float ps[CS][LHS ? P2 : 1];
-    __shared__ double sh[2 * WS + 6];
     __shared__ RT term[WS > 1 ? WSMAX * 2 * R * 128 : 1];  // [WFS][node of the thread][thread]
     const int l = by, s0 = J.s0 + bz * CS, ns = min(CS, J.s0 + J.nsys - s0);
     const int nxl = G.xnx[l], nyl = G.xny[l];
@@ -1255,12 +1273,12 @@ __global__ __launch_bounds__(128 * WS) void k_layer_m8(KARGS, int psel_, int ose
                 for (int k = 0; k <= R; k++) {
                     const RT qa = bload<RT>(rs, ca + ro[k]), qb = bload<RT>(rs, cb + ro[k]),
                              qc = bload<RT>(rs, cc + ro[k]);
-                    h0[k] = gx * qb + fx * qa;
-                    h1[k] = gx * qc + fx * qb;
+                    h0[k] = lerp2(fx, qa, gx, qb);
+                    h1[k] = lerp2(fx, qb, gx, qc);
                 }
 #pragma unroll
                 for (int r = 0; r < R; r++) {
-                    const RT c0 = fy * h0[r] + gy * h0[r + 1], c1 = fy * h1[r] + gy * h1[r + 1];
+                    const RT c0 = lerp2(fy, h0[r], gy, h0[r + 1]), c1 = lerp2(fy, h1[r], gy, h1[r + 1]);
                     if constexpr (WS > 1) {
                         tm[r * 128] = c0;
                         tm[(R + r) * 128] = c1;
@@ -1281,18 +1299,16 @@ __global__ __launch_bounds__(128 * WS) void k_layer_m8(KARGS, int psel_, int ose
 #pragma unroll
                     for (int r = 0; r < R; r++) acc[0][c][r] += term[w * (2 * R * 128) + (c * R + r) * 128 + tid];
     }
-    double dot[CS];
+    if (grp != 0) return;
 #pragma unroll
     for (int si = 0; si < CS; si++) {
-        dot[si] = 0;
-        if (si < ns && grp == 0) {
+        double dr[R];
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            double d[2] = {0, 0};
 #pragma unroll
             for (int c = 0; c < 2; c++) {
-                if (c >= nc) continue;
-#pragma unroll
-                for (int r = 0; r < R; r++) {
-                    if (r >= nr) continue;
-                    const int jy = jyb + r;
+                if (si < ns && c < nc && r < nr) {
                     RT a = acc[si][c][r];
                     if (LHS) {
                         const float *P0 = ps[si] + (R * ty + r + 2) * PW + 2 * tx + c + 2;
@@ -1302,20 +1318,28 @@ __global__ __launch_bounds__(128 * WS) void k_layer_m8(KARGS, int psel_, int ose
                         const RT sd = P(-1, -1) + P(1, -1) + P(-1, 1) + P(1, 1);
                         const RT s2 = P(-2, 0) + P(2, 0) + P(0, -2) + P(0, 2);
                         a += (RT)G.l2c[l] * (RT(20) * cv - RT(8) * s4 + RT(2) * sd + s2);
-                        dot[si] = dfma(cv, a, dot[si], G.dot32);
+                        d[c] = dmul(cv, a, G.dot32);
                     } else {
-                        dot[si] = dfma(a, a, dot[si], G.dot32);
+                        d[c] = dmul(a, a, G.dot32);
                     }
-                    out[(long)(s0 + si) * G.nxtot + G.xoff[l] + jy * nxl + jx + c] = a;
+                    out[(long)(s0 + si) * G.nxtot + G.xoff[l] + (jyb + r) * nxl + jx + c] = a;
                 }
             }
+            dr[r] = dadd(d[0], d[1], G.dot32);
         }
-    }
-#pragma unroll
-    for (int si = 0; si < CS; si++) {
-        const double d = block_sum(dot[si], sh, G.dot32);
-        if (threadIdx.x == 0 && part && si < ns)
-            part[(long)(s0 + si) * partstride + by * PD.ltiles + bx] = d;
+        // strips of 4 rows (the layer tile sums above), then 4 strips a tile:
+        // a wave holds LT / 2 rows, i.e. one 16 x 16 tile or two
+        double d = dadd(dr[0], dr[1], G.dot32);
+        if constexpr (R == 4) d = dadd(d, dadd(dr[2], dr[3], G.dot32), G.dot32);
+        else d = dadd(d, __shfl_xor(d, 8, 64), G.dot32);
+        for (int o : {1, 2, 4}) d = dadd(d, __shfl_xor(d, o, 64), G.dot32);
+        constexpr int SL = 32 / R;  // lanes of a strip
+        double t = d;
+        for (int k = 1; k < 4; k++) t = dadd(t, __shfl_down(d, SL * k, 64), G.dot32);
+        const int lane = threadIdx.x & 63, half = (tid >> 6) * (LT / 32) + lane / (4 * SL);
+        const int ty1 = (bx / ntx) * (LT / 16) + half;  // row of 16 x 16 tiles
+        if (lane % (4 * SL) == 0 && active && part && si < ns && ty1 < (nyl + TILE - 1) / TILE)
+            part[(long)(s0 + si) * partstride + by * PD.ltiles + ty1 * ntx + bx % ntx] = t;
     }
 }
 

@@ -73,7 +73,6 @@ struct Geom {
     const int4 *hxt_x, *hxt_y;    // per (w,l) per layer index: up to 4 ploc indices (-1 pad)
     long hxt_xoff[MAXL + 1];      // offset of layer l in a (w,*) transposed x table
     int matched;                  // every (w,l) ray is matched sampling (fast path)
-    int lty;                      // layer tile height: TILE, or LTY / LTY2 (k_layer_m8)
     const MRay *mray;             // [w*MAXL + l]
     // subapertures
     const int *saidx;             // per WFS per ploc point: subaperture with that lower-left corner, -1
@@ -153,7 +152,7 @@ struct PlanDev {
     float2 *speci;      // inverse spectrum
     Scal SC;
     int *stop;
-    int ltiles;         // layer tiles per layer (layer partial index stride)
+    int ltiles;         // TILE x TILE tiles per layer (layer partial index stride)
     // TT removal inside the LHS (ptt_lhs): the operator's own gradients
     // G HX p (residual precision, ngtot per system) and their TT projection
     // PTT G HX p (FP64, 2 per system and WFS); null otherwise

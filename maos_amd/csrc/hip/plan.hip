@@ -121,6 +121,7 @@ struct Sub {
     int nthr = 0; // its threads per workgroup
     int regL = 0; // its lanes per column FFT (shL of every job)
     bool split = false;  // WFS and layer stages: the split form
+    int lty = TILE;      // layer stage: tile rows
     size_t lds = 0;
     DevBuf<WGI> wgi;
     int nwg = 0;
@@ -216,7 +217,7 @@ struct gpu_tomo {
     // systems per workgroup chosen by the autotuner (0: heuristic)
     int tune_wfs = 0, tune_layer = 0, tune_col = 0;
     long gen = 0;         // bumped whenever the launch tables must be rebuilt (shape, precision)
-    int tune_lty = 0;     // layer tile rows: 0 = built-in choice (default_lty), TILE, LTY2 or LTY
+    int tune_lty = 0;     // layer tile rows: 0 = built-in choice (layer_rows), TILE, LTY2 or LTY
     int tune_colfft = 0;  // column kernel: 0 = registers where available, 1 = registers, 2 = LDS stages
     bool colr_ok = false; // the register column kernel applies (per-frequency blocks, ny = shL x shP)
     bool lty_ok = false;  // LTY-row tiles fit every layer of this (matched) plan
@@ -440,18 +441,20 @@ void build_mreg(gpu_tomo *g, const std::vector<float2> &hM, const std::vector<in
     g->grp_blk_host = hgb;
 }
 
-// Layer tile rows of a matched plan without a tuned choice, from its own sizes
-// (a plan computes the same bits in every call).  Layers above LTY rows:
-// LTY2 (k_layer of the 30 m system, 64 / 32 / 16 rows at one system per
-// workgroup: 1 system 9.7 8.1 7.4, 32: 19.8 17.7 30.9, 256: 90 89 200 us).
-// Smaller ones: TILE rows for few systems, LTY2 from about 160 000 nodes in
-// the plan on (16 / 32 rows; 20 m of 4 layers, 16 384 nodes: 1 system 6.4 7.0,
-// 16: 8.0 7.4, 64: 19.5 11.8, 256: 61 29; 10 m, 5184 nodes: 16: 5.9 6.3, 32:
-// 7.1 6.5, 64: 10.5 7.6, 256: 25.5 15.2 us).
-constexpr long LTY2_NODES = 160000;
-int default_lty(const gpu_tomo *g) {
-    if (g->lty_ok) return LTY2;
-    return g->lty2_ok && g->G.nxtot * g->nbatch >= LTY2_NODES ? LTY2 : TILE;
+// Layer tile rows for nsys systems of a plan (the shape does not change
+// results: p.Ap is summed per 16 x 16 nodes in one order).  Without a tuned
+// choice: TILE rows, in the split form where that applies, for a few small
+// systems, LTY2 from about 100 000 nodes in the launch on.  k_layer, us, 16 / 32
+// rows (64): 5184 nodes a system, 1 system 4.8 5.4, 16: 5.7 6.3, 32: 7.0 6.2,
+// 256: 25.9 15.1; 6272 nodes, 16: 6.2 5.6; 16 384 nodes, 1: 5.1 5.6, 8: 6.1
+// 5.6, 64: 19.7 11.3; the 30 m system, 1: 5.7 6.1 (12.4), 8: 11.4 8.5 (12.4),
+// 32: 31.3 17.5 (19.3), 256: 201 88 (91).
+constexpr long LTY2_NODES = 100000;
+int layer_rows(const gpu_tomo *g, int nsys) {
+    if (!g->G.matched || g->tune_lty == TILE) return TILE;
+    if (g->tune_lty == LTY) return g->lty_ok ? LTY : TILE;
+    if (!g->lty2_ok) return TILE;
+    return g->tune_lty == LTY2 || g->G.nxtot * nsys >= LTY2_NODES ? LTY2 : TILE;
 }
 
 void build_plan(gpu_tomo *g, const mt_recon_t *R) {
@@ -628,7 +631,6 @@ void build_plan(gpu_tomo *g, const mt_recon_t *R) {
         }
     // the matched kernels wrap the L2 window once: layers of at least TILE + 2
     // (16 x 16 tiles), LTY2 + 2 (16 x 32) or LTY + 2 rows (16 x 64 tiles)
-    G.lty = TILE;
     for (int l = 0; l < R->npsr; l++)
         if (R->xnx[l] < TILE + 2 || R->xny[l] < TILE + 2) matched = 0;
     g->lty_ok = g->lty2_ok = matched != 0;
@@ -637,7 +639,6 @@ void build_plan(gpu_tomo *g, const mt_recon_t *R) {
         if (R->xny[l] < LTY2 + 2) g->lty2_ok = false;
     }
     G.matched = matched;
-    if (matched) G.lty = default_lty(g);
     g->mray.upload(hm);
     G.mray = g->mray.p;
     g->hx_nx.upload(hnx);
@@ -914,33 +915,18 @@ void build_plan(gpu_tomo *g, const mt_recon_t *R) {
     if (G.precond && row_lds(G.fnx, 1) > 64 * 1024) fail(MT_EINVAL, "layer grid too large for the row FFT kernel");
 }
 
-// Tiles of the layer passes (the largest layer decides; all layers are
-// equal when FDPCG is used).
-int layer_tiles(const Geom &G) {
+// Tiles of the layer passes with lty rows (the largest layer decides; all
+// layers are equal when FDPCG is used).
+int layer_tiles(const Geom &G, int lty = TILE) {
     int t = 1;
     for (int l = 0; l < G.npsr; l++)
-        t = std::max(t, ((G.xnx[l] + TILE - 1) / TILE) * ((G.xny[l] + G.lty - 1) / G.lty));
+        t = std::max(t, ((G.xnx[l] + TILE - 1) / TILE) * ((G.xny[l] + lty - 1) / lty));
     return t;
 }
 
 void upload_plandev(gpu_tomo *g);
 void upload_plandev(gpu_tomo *g, hipStream_t st);
 void drop_batches(gpu_tomo *g);
-// Apply the layer tile height choice (the plan's device record and
-// partial counts follow; launch tables are rebuilt on next use).
-void apply_lty(gpu_tomo *g) {
-    if (!g->G.matched) return;
-    const int lty = g->tune_lty == TILE   ? TILE
-                    : g->tune_lty == LTY2 ? (g->lty2_ok ? LTY2 : TILE)
-                    : g->tune_lty == LTY  ? (g->lty_ok ? LTY : TILE)
-                                          : default_lty(g);
-    if (lty == g->G.lty) return;
-    g->G.lty = lty;
-    g->SC.npart_layer = layer_tiles(g->G) * g->G.npsr;
-    upload_plandev(g);
-    drop_batches(g);
-}
-
 void upload_plandev(gpu_tomo *g, hipStream_t st) {
     PlanDev h{};
     h.G = g->G;
@@ -984,9 +970,7 @@ void alloc_state(gpu_tomo *g) {
     }
     g->specf.alloc(ns * std::max<long>(G.nspec, 1));
     g->speci.alloc(ns * std::max<long>(G.nspec, 1));
-    Geom g16 = G;  // partials sized for the smaller layer tiles (either height may be chosen later)
-    g16.lty = TILE;
-    const int maxpart = std::max({layer_tiles(g16) * G.npsr, G.nrowblk, G.ngroup, 1});
+    const int maxpart = std::max({layer_tiles(G) * G.npsr, G.nrowblk, G.ngroup, 1});
     g->part_pap.alloc(ns * maxpart);
     g->part_rz.alloc(ns * maxpart);
     g->part_rr.alloc(ns * maxpart);
@@ -1264,14 +1248,17 @@ std::unique_ptr<Batch> make_batch(const std::vector<gpu_tomo *> &plans, const st
                 });
     build_stage(b, b.layer,
                 [&](int j, std::vector<int> &k) {
-                    k = {G(j).matched ? (G(j).lty == LTY ? 2 : G(j).lty == LTY2 ? 3 : 1) : 0};
+                    const int lty = layer_rows(b.plan[j], NS(j));
+                    k = {G(j).matched ? (lty == LTY ? 2 : lty == LTY2 ? 3 : 1) : 0};
                     return true;
                 },
                 [&](const Sub &sb, int j) {
-                    return JobGrid{layer_tiles(G(j)), G(j).npsr, sb.matched ? ceil_div(NS(j), sb.cs) : NS(j)};
+                    return JobGrid{layer_tiles(G(j), sb.lty), G(j).npsr, sb.matched ? ceil_div(NS(j), sb.cs) : NS(j)};
                 },
                 [&](Sub &sb, const std::vector<int> &k, const std::vector<int> &js) {
                     sb.matched = k[0];
+                    sb.lty = k[0] == 2 ? LTY : k[0] == 3 ? LTY2 : TILE;
+                    auto tiles = [&](int j) { return (long)layer_tiles(G(j), sb.lty) * G(j).npsr; };
                     const int tuned = b.plan[js[0]]->tune_layer;
                     sb.cs = !sb.matched ? 1
                             : tuned     ? tuned
@@ -1279,12 +1266,9 @@ std::unique_ptr<Batch> make_batch(const std::vector<gpu_tomo *> &plans, const st
                             // tiles, 1 / 2 / 4 systems: 32: 17.7 18.6 23.5, 256: 89 91 98 us).
                             // k_layer_m: two once that leaves 1024 workgroups (10 m of 4 layers:
                             // 32: 7.1 8.0 10.3, 64: 10.5 9.4 11.8, 256: 25.5 20.8 20.5)
-                            : G(js[0]).lty != TILE
-                                ? 1
-                                : pick_cs(jw_of(js, [&](int j) { return (long)layer_tiles(G(j)) * G(j).npsr; }),
-                                          2, 1024, 1024);
-                    sb.split = sb.matched && sb.cs == 1 && can_split(js) && G(js[0]).lty != LTY &&
-                               wgs(js, [&](int j) { return (long)layer_tiles(G(j)) * G(j).npsr; }) <= SPLIT_WGS;
+                            : sb.lty != TILE ? 1
+                                             : pick_cs(jw_of(js, tiles), 2, 1024, 1024);
+                    sb.split = sb.matched && sb.cs == 1 && can_split(js) && sb.lty != LTY && wgs(js, tiles) <= SPLIT_WGS;
                 });
     if (b.precond) {
         build_stage(b, b.row, [&](int j, std::vector<int> &k) { k = row_key(j); return true; },
@@ -1673,9 +1657,7 @@ struct NoallocLayout {
 NoallocLayout noalloc_layout(const gpu_tomo *g) {
     const Geom &G = g->G;
     const size_t rt = g->rt64 ? 8 : 4, sp = g->spec64 ? 16 : 8;
-    Geom g16 = G;
-    g16.lty = TILE;
-    const size_t maxpart = (size_t)std::max({layer_tiles(g16) * G.npsr, G.nrowblk, G.ngroup, 1});
+    const size_t maxpart = (size_t)std::max({layer_tiles(G) * G.npsr, G.nrowblk, G.ngroup, 1});
     NoallocLayout L{};
     size_t o = 0;
     auto take = [&](size_t bytes) {
@@ -2022,9 +2004,7 @@ int gpu_tomo_solve_dev_noalloc(gpu_tomo_t *g, const float *d_grad, float *d_x, d
                                 " bytes available");
         hipStream_t st = stream ? (hipStream_t)stream : g->stream;
         const Geom &G = g->G;
-        Geom g16 = G;
-        g16.lty = TILE;
-        const int maxpart = std::max({layer_tiles(g16) * G.npsr, G.nrowblk, G.ngroup, 1});
+        const int maxpart = std::max({layer_tiles(G) * G.npsr, G.nrowblk, G.ngroup, 1});
         for (int s = 0; s < nsys; s++) {
             // a system at a time through the one-system tables; the
             // workspace is reused, in stream order
@@ -2404,7 +2384,6 @@ void group_apply(gpu_tomo_group *grp, const int *c) {
         g->tune_lty = c[3];
         g->tune_colfft = c[4];
         drop_batches(g);
-        apply_lty(g);
         noalloc_init(g);
     }
     group_rebuild(grp);
@@ -2492,7 +2471,6 @@ int gpu_tomo_tune_set(gpu_tomo_t *g, const int *choice) {
         g->tune_colfft = choice[4];
         g->tune_flights = choice[5];
         drop_batches(g);
-        apply_lty(g);
         noalloc_init(g);
     });
 }
@@ -2534,12 +2512,11 @@ int gpu_tomo_autotune(gpu_tomo_t *g, int nsys, int *choice) {
         // they fit) and systems per workgroup together
         {
             double best = 1e30;
-            int bestl = g->G.lty, bestc = 1;
+            int bestl = layer_rows(g, nsys), bestc = 1;
             for (int lty : {LTY, LTY2, TILE}) {
                 if (lty == LTY && !(g->G.matched && g->lty_ok)) continue;
                 if (lty == LTY2 && !(g->G.matched && g->lty2_ok)) continue;
                 g->tune_lty = lty;
-                apply_lty(g);
                 for (int c = 1; c <= 4; c <<= 1) {
                     g->tune_layer = c;
                     const double t = stage_ms(KC_LAYER);
@@ -2552,7 +2529,6 @@ int gpu_tomo_autotune(gpu_tomo_t *g, int nsys, int *choice) {
             }
             g->tune_lty = bestl;
             g->tune_layer = bestc;
-            apply_lty(g);
         }
         // the column stage: register kernel (where it applies; one system
         // per lane group, no systems-per-workgroup choice) or the LDS kernel
@@ -2633,7 +2609,7 @@ int gpu_tomo_autotune(gpu_tomo_t *g, int nsys, int *choice) {
             choice[0] = g->tune_wfs;
             choice[1] = g->tune_layer;
             choice[2] = g->tune_col;
-            choice[3] = g->G.lty;
+            choice[3] = layer_rows(g, nsys);
             choice[4] = g->tune_colfft;
             choice[5] = g->tune_flights;
         }
