@@ -27,7 +27,7 @@ constexpr int TILE = 16;      // output tile edge of the WFS / layer passes
 constexpr int TAPS = 4;       // max ploc samples landing on one layer node per axis
 constexpr int ROWS = 16;      // rows per row-FFT workgroup (8 complex FFTs)
 constexpr int LTY = 64;       // tile height of the 16 x 64 layer kernel (k_layer_m8)
-constexpr int LTY2 = 32;      // tile height of its 16 x 32 form
+constexpr int LTY2 = 32;      // of its 16 x 32 form
 constexpr int MAXN = 1024;    // largest FFT length (layer grid edge)
 
 // Matched-sampling ray of one (WFS, layer) pair: ploc index i maps to layer
