@@ -107,6 +107,12 @@ struct D64 {
     const int *txp, *typ, *txi, *tyi;
     const double *txw, *tyw;
     int txo[X64W * X64L], tyo[X64W * X64L];
+    // the same where no node takes more than two rays (taps2): per (k, l) and
+    // node, at k axo[npsr] + axo[l] + node, the ploc indices (-1: none)
+    int taps2;
+    int axo[X64L + 1], ayo[X64L + 1];  // prefix sums of lnx, lny
+    const int2 *t2xi, *t2yi;
+    const double2 *t2xw, *t2yw;
     // GP of WFS k: rows (CSR, pointer array at rpo[k]) and columns (CSC,
     // pointer array at cpo[k]); entry indices absolute
     const long *grp, *gri, *gcp, *gci;
@@ -167,6 +173,37 @@ __device__ __forceinline__ double *prt(const D64 &D, int s) { return D.part + (l
 // Operators
 // ---------------------------------------------------------------------------
 
+// The loads of these gathers depend on index loads, and one system has few
+// workgroups, so a pass is bound by that latency chain: CH64 WFSs, layers or
+// matrix entries are loaded at a time (indices clamped, terms that are not there
+// left out when they are added), in the order of the plain loop.  30 m system,
+// one system, us a launch: k64_hx 7.3 -> 5.5, k64_gpt 5.7 -> 4.5, k64_grad and
+// k64_wg 8.2 -> k64_gw 4.4, k64_hxt 14.4 -> 7.5; the solve 2290 -> 1950.
+constexpr int CH64 = 3;
+
+// sum over e in [e0, e1) of val[e] src[idx[e]]
+__device__ __forceinline__ double gather64(const long *__restrict__ idx, const double *__restrict__ val, long e0,
+                                           long e1, const double *__restrict__ src) {
+    constexpr int C = 4;
+    double acc = 0;
+    for (long e = e0; e < e1; e += C) {
+        double w[C], v[C];
+        long i[C];
+#pragma unroll
+        for (int u = 0; u < C; u++) {
+            const long eu = e + u < e1 ? e + u : e1 - 1;
+            i[u] = idx[eu];
+            w[u] = val[eu];
+        }
+#pragma unroll
+        for (int u = 0; u < C; u++) v[u] = src[i[u]];
+#pragma unroll
+        for (int u = 0; u < C; u++)
+            if (e + u < e1) acc += w[u] * v[u];
+    }
+    return acc;
+}
+
 // opd_k = HX_k v (prop_grid_stat, lib/prop_grid.c:47-343).  Grid (ploc
 // chunks, WFS, systems); v: per-system layer vectors, stride nxtot.
 __global__ __launch_bounds__(B64) void k64_hx(const D64 *__restrict__ Dp, const double *__restrict__ v, int ws0) {
@@ -177,16 +214,33 @@ __global__ __launch_bounds__(B64) void k64_hx(const D64 *__restrict__ Dp, const 
     const int iy = (int)(pt / D.pnx), ix = (int)(pt - (long)iy * D.pnx);
     const double *src = v + (long)z * D.nxtot;
     double acc = 0;
-    for (int l = 0; l < D.npsr; l++) {
-        const long kl = (long)k * D.npsr + l;
-        const int2 a = D.rnx[kl * D.pnx + ix], b = D.rny[kl * D.pny + iy];
-        if (a.x < 0 || b.x < 0) continue;
-        const double fx = D.rfx[kl * D.pnx + ix], fy = D.rfy[kl * D.pny + iy];
-        const double *m = src + D.loff[l];
-        const int nx = D.lnx[l];
-        const double v00 = m[(long)b.x * nx + a.x], v01 = m[(long)b.x * nx + a.y];
-        const double v10 = m[(long)b.y * nx + a.x], v11 = m[(long)b.y * nx + a.y];
-        acc += (1 - fy) * ((1 - fx) * v00 + fx * v01) + fy * ((1 - fx) * v10 + fx * v11);
+    for (int l0 = 0; l0 < D.npsr; l0 += CH64) {
+        int2 a[CH64], b[CH64];
+        double fx[CH64], fy[CH64], v00[CH64], v01[CH64], v10[CH64], v11[CH64];
+#pragma unroll
+        for (int u = 0; u < CH64; u++) {
+            const long kl = (long)k * D.npsr + min(l0 + u, D.npsr - 1);
+            a[u] = D.rnx[kl * D.pnx + ix];
+            b[u] = D.rny[kl * D.pny + iy];
+            fx[u] = D.rfx[kl * D.pnx + ix];
+            fy[u] = D.rfy[kl * D.pny + iy];
+        }
+#pragma unroll
+        for (int u = 0; u < CH64; u++) {
+            const int l = min(l0 + u, D.npsr - 1);
+            const double *m = src + D.loff[l];
+            const long r0 = (long)max(b[u].x, 0) * D.lnx[l], r1 = (long)max(b[u].y, 0) * D.lnx[l];
+            const int c0 = max(a[u].x, 0), c1 = max(a[u].y, 0);
+            v00[u] = m[r0 + c0];
+            v01[u] = m[r0 + c1];
+            v10[u] = m[r1 + c0];
+            v11[u] = m[r1 + c1];
+        }
+#pragma unroll
+        for (int u = 0; u < CH64; u++)
+            if (l0 + u < D.npsr && a[u].x >= 0 && b[u].x >= 0)
+                acc += (1 - fy[u]) * ((1 - fx[u]) * v00[u] + fx[u] * v01[u]) +
+                       fy[u] * ((1 - fx[u]) * v10[u] + fx[u] * v11[u]);
     }
     D.opd[((long)s * D.nw + k) * D.nploc + pt] = acc;
 }
@@ -209,7 +263,7 @@ __global__ __launch_bounds__(B64) void k64_grad(const D64 *__restrict__ Dp, int 
         if (FROM_OPD) {
             const double *opd = D.opd + ((long)s * D.nw + k) * D.nploc;
             const long *rp = D.grp + D.rpo[k];
-            for (long e = rp[i]; e < rp[i + 1]; e++) gv += D.grx[e] * opd[D.gri[e]];
+            gv = gather64(D.gri, D.grx, rp[i], rp[i + 1], opd);
             D.g[o] = gv;
         } else {
             gv = D.gin[o];
@@ -251,6 +305,25 @@ __global__ __launch_bounds__(B64) void k64_wg(const D64 *__restrict__ Dp, int ws
     D.wg[o + nsa + i] = ne[2] * gx + ne[1] * gy;
 }
 
+// wg = NEA^-1 GP opd_k per subaperture, where the LHS removes no TT (k64_grad
+// and k64_wg in one launch).  Grid (chunks of nsa, WFS, systems).
+__global__ __launch_bounds__(B64) void k64_gw(const D64 *__restrict__ Dp, int ws0) {
+    const D64 &D = *Dp;
+    const int k = blockIdx.y, s = ws0 + blockIdx.z;
+    const long nsa = D.nsa[k];
+    const long i = (long)blockIdx.x * B64 + threadIdx.x;
+    if (i >= nsa) return;
+    const double *opd = D.opd + ((long)s * D.nw + k) * D.nploc;
+    const long *rp = D.grp + D.rpo[k];
+    const long ex0 = rp[i], ex1 = rp[i + 1], ey0 = rp[nsa + i], ey1 = rp[nsa + i + 1];
+    const double *ne = D.neai + 3 * (D.saoff[k] + i);
+    const double n0 = ne[0], n1 = ne[1], n2 = ne[2];
+    const double gx = gather64(D.gri, D.grx, ex0, ex1, opd), gy = gather64(D.gri, D.grx, ey0, ey1, opd);
+    const long o = (long)s * D.ngtot + D.goff[k];
+    D.wg[o + i] = n0 * gx + n2 * gy;
+    D.wg[o + nsa + i] = n2 * gx + n1 * gy;
+}
+
 // q_k = GP_k' wg_k (column gather of the CSC form).  Grid (ploc chunks, WFS,
 // systems).
 __global__ __launch_bounds__(B64) void k64_gpt(const D64 *__restrict__ Dp, int ws0) {
@@ -260,16 +333,15 @@ __global__ __launch_bounds__(B64) void k64_gpt(const D64 *__restrict__ Dp, int w
     if (pt >= D.nploc) return;
     const long *cp = D.gcp + D.cpo[k];
     const double *wg = D.wg + (long)s * D.ngtot + D.goff[k];
-    double acc = 0;
-    for (long e = cp[pt]; e < cp[pt + 1]; e++) acc += D.gcx[e] * wg[D.gci[e]];
-    D.q[((long)s * D.nw + k) * D.nploc + pt] = acc;
+    D.q[((long)s * D.nw + k) * D.nploc + pt] = gather64(D.gci, D.gcx, cp[pt], cp[pt + 1], wg);
 }
 
 // out = sum_k HX_k' q_k; LHS adds L2' L2 v (two periodic 5-point passes,
 // lib/laplacian.c:70-97, composed at the node) and writes the workgroup's
 // partial of v . out.  Grid (node chunks, systems); v, out: per-system
-// vectors of stride nxtot.
-template <bool LHS>
+// vectors of stride nxtot.  T2: at most two rays a node and axis (any plan whose
+// layers are no coarser than ploc along the rays); else the lists.
+template <bool LHS, bool T2>
 __global__ __launch_bounds__(B64) void k64_hxt(const D64 *__restrict__ Dp, const double *__restrict__ v,
                                                double *__restrict__ out, int ws0) {
     const D64 &D = *Dp;
@@ -284,6 +356,44 @@ __global__ __launch_bounds__(B64) void k64_hxt(const D64 *__restrict__ Dp, const
         const int nx = D.lnx[l], ny = D.lny[l];
         const long rem = n - D.loff[l];
         const int iy = (int)(rem / nx), ix = (int)(rem - (long)iy * nx);
+        if constexpr (T2) {
+            const int2 *xi = D.t2xi + D.axo[l] + ix, *yi = D.t2yi + D.ayo[l] + iy;
+            const double2 *xw = D.t2xw + D.axo[l] + ix, *yw = D.t2yw + D.ayo[l] + iy;
+            const int sx = D.axo[D.npsr], sy = D.ayo[D.npsr];
+            for (int k0 = 0; k0 < D.nw; k0 += CH64) {
+                int2 jx[CH64], jy[CH64];
+                double2 wx[CH64], wy[CH64];
+                double q00[CH64], q01[CH64], q10[CH64], q11[CH64];
+#pragma unroll
+                for (int u = 0; u < CH64; u++) {
+                    const int k = min(k0 + u, D.nw - 1);
+                    jx[u] = xi[(long)k * sx];
+                    jy[u] = yi[(long)k * sy];
+                    wx[u] = xw[(long)k * sx];
+                    wy[u] = yw[(long)k * sy];
+                }
+#pragma unroll
+                for (int u = 0; u < CH64; u++) {
+                    const double *q = D.q + ((long)s * D.nw + min(k0 + u, D.nw - 1)) * D.nploc;
+                    const long r0 = (long)max(jy[u].x, 0) * D.pnx, r1 = (long)max(jy[u].y, 0) * D.pnx;
+                    const int c0 = max(jx[u].x, 0), c1 = max(jx[u].y, 0);
+                    q00[u] = q[r0 + c0];
+                    q01[u] = q[r0 + c1];
+                    q10[u] = q[r1 + c0];
+                    q11[u] = q[r1 + c1];
+                }
+#pragma unroll
+                for (int u = 0; u < CH64; u++) {
+                    if (k0 + u >= D.nw) break;
+                    // a tap that is not there adds 0 (never 0 times a value)
+                    const bool x0 = jx[u].x >= 0, x1 = jx[u].y >= 0, y0 = jy[u].x >= 0, y1 = jy[u].y >= 0;
+                    acc += wx[u].x * wy[u].x * (x0 && y0 ? q00[u] : 0.0);
+                    acc += wx[u].y * wy[u].x * (x1 && y0 ? q01[u] : 0.0);
+                    acc += wx[u].x * wy[u].y * (x0 && y1 ? q10[u] : 0.0);
+                    acc += wx[u].y * wy[u].y * (x1 && y1 ? q11[u] : 0.0);
+                }
+            }
+        } else
         for (int k = 0; k < D.nw; k++) {
             const int kl = k * D.npsr + l;
             const int x0 = D.txp[D.txo[kl] + ix], x1 = D.txp[D.txo[kl] + ix + 1];
@@ -600,6 +710,8 @@ struct tomo64 {
     Buf<double> rfx, rfy;
     Buf<int> txp, typ, txi, tyi;
     Buf<double> txw, tyw;
+    Buf<int2> t2xi, t2yi;
+    Buf<double2> t2xw, t2yw;
     Buf<long> grp, gri, gcp, gci;
     Buf<double> grx, gcx, neai, ptt;
     Buf<double2> twx, twy, Minv;
@@ -728,6 +840,14 @@ void build64(tomo64 *t, const mt_recon_t *R, int nbatch) {
     std::vector<double> hfx(hnx.size()), hfy(hny.size());
     std::vector<int> htxp, htyp, htxi, htyi;
     std::vector<double> htxw, htyw;
+    std::vector<int2> h2xi, h2yi;
+    std::vector<double2> h2xw, h2yw;
+    D.taps2 = 1;
+    D.axo[0] = D.ayo[0] = 0;
+    for (int l = 0; l < D.npsr; l++) {
+        D.axo[l + 1] = D.axo[l] + D.lnx[l];
+        D.ayo[l + 1] = D.ayo[l] + D.lny[l];
+    }
     for (int k = 0; k < nw; k++) {
         const int w = t->active[k];
         for (int l = 0; l < D.npsr; l++) {
@@ -746,8 +866,8 @@ void build64(tomo64 *t, const mt_recon_t *R, int nbatch) {
                 hny[kl * pny + i] = ay.nn[i];
                 hfy[kl * pny + i] = ay.f[i];
             }
-            auto transpose = [](const mtk::Axis &a, int nnode, std::vector<int> &ptr, std::vector<int> &idx,
-                                std::vector<double> &wt) {
+            auto transpose = [&D](const mtk::Axis &a, int nnode, std::vector<int> &ptr, std::vector<int> &idx,
+                                  std::vector<double> &wt, std::vector<int2> &i2, std::vector<double2> &w2) {
                 std::vector<std::vector<std::pair<int, double>>> lists(nnode);
                 for (size_t i = 0; i < a.nn.size(); i++) {
                     if (a.nn[i].x < 0) continue;
@@ -760,23 +880,34 @@ void build64(tomo64 *t, const mt_recon_t *R, int nbatch) {
                         idx.push_back(e.first);
                         wt.push_back(e.second);
                     }
+                    const auto &L = lists[n];
+                    if (L.size() > 2) D.taps2 = 0;
+                    i2.push_back(make_int2(L.size() > 0 ? L[0].first : -1, L.size() > 1 ? L[1].first : -1));
+                    w2.push_back(make_double2(L.size() > 0 ? L[0].second : 0, L.size() > 1 ? L[1].second : 0));
                 }
                 ptr.push_back((int)idx.size());
             };
-            transpose(ax, D.lnx[l], htxp, htxi, htxw);
-            transpose(ay, D.lny[l], htyp, htyi, htyw);
+            transpose(ax, D.lnx[l], htxp, htxi, htxw, h2xi, h2xw);
+            transpose(ay, D.lny[l], htyp, htyi, htyw, h2yi, h2yw);
         }
     }
     t->rnx.upload(hnx);
     t->rny.upload(hny);
     t->rfx.upload(hfx);
     t->rfy.upload(hfy);
-    t->txp.upload(htxp);
-    t->typ.upload(htyp);
-    t->txi.upload(htxi);
-    t->tyi.upload(htyi);
-    t->txw.upload(htxw);
-    t->tyw.upload(htyw);
+    if (D.taps2) {
+        t->t2xi.upload(h2xi);
+        t->t2yi.upload(h2yi);
+        t->t2xw.upload(h2xw);
+        t->t2yw.upload(h2yw);
+    } else {
+        t->txp.upload(htxp);
+        t->typ.upload(htyp);
+        t->txi.upload(htxi);
+        t->tyi.upload(htyi);
+        t->txw.upload(htxw);
+        t->tyw.upload(htyw);
+    }
     // GP: CSC as given, CSR by transposition
     std::vector<long> hcp, hci, hrp, hri;
     std::vector<double> hcx, hrx;
@@ -879,6 +1010,10 @@ void build64(tomo64 *t, const mt_recon_t *R, int nbatch) {
     D.tyi = t->tyi.p;
     D.txw = t->txw.p;
     D.tyw = t->tyw.p;
+    D.t2xi = t->t2xi.p;
+    D.t2yi = t->t2yi.p;
+    D.t2xw = t->t2xw.p;
+    D.t2yw = t->t2yw.p;
     D.grp = t->grp.p;
     D.gri = t->gri.p;
     D.grx = t->grx.p;
@@ -917,22 +1052,31 @@ void build64(tomo64 *t, const mt_recon_t *R, int nbatch) {
 dim3 g_ploc(const D64 &D, int n) { return dim3((unsigned)((D.nploc + B64 - 1) / B64), D.nw, n); }
 dim3 g_node(const D64 &D, int n) { return dim3(D.nch, n); }
 
+template <bool LHS>
+void launch_hxt(tomo64 *t, hipStream_t st, const double *v, double *out, int ws0, int n) {
+    if (t->H.taps2) hipLaunchKernelGGL((k64_hxt<LHS, true>), g_node(t->H, n), dim3(B64), 0, st, t->dev.p, v, out, ws0);
+    else hipLaunchKernelGGL((k64_hxt<LHS, false>), g_node(t->H, n), dim3(B64), 0, st, t->dev.p, v, out, ws0);
+}
 // out = HX' GP' W (I - TT PTT) gin (TomoR, without the alpha scale)
 void enq_R(tomo64 *t, hipStream_t st, double *out, int ws0, int n) {
     const D64 &D = t->H;
     hipLaunchKernelGGL(k64_grad<false>, dim3(D.nchg, D.nw, n), dim3(B64), 0, st, t->dev.p, ws0);
     hipLaunchKernelGGL(k64_wg<false>, dim3(D.nchs, D.nw, n), dim3(B64), 0, st, t->dev.p, ws0);
     hipLaunchKernelGGL(k64_gpt, g_ploc(D, n), dim3(B64), 0, st, t->dev.p, ws0);
-    hipLaunchKernelGGL(k64_hxt<false>, g_node(D, n), dim3(B64), 0, st, t->dev.p, (const double *)nullptr, out, ws0);
+    launch_hxt<false>(t, st, nullptr, out, ws0, n);
 }
 // out = (HX' GP' W GP HX + L2'L2) v and the partials of v . out
 void enq_L(tomo64 *t, hipStream_t st, const double *v, double *out, int ws0, int n) {
     const D64 &D = t->H;
     hipLaunchKernelGGL(k64_hx, g_ploc(D, n), dim3(B64), 0, st, t->dev.p, v, ws0);
-    hipLaunchKernelGGL(k64_grad<true>, dim3(D.nchg, D.nw, n), dim3(B64), 0, st, t->dev.p, ws0);
-    hipLaunchKernelGGL(k64_wg<true>, dim3(D.nchs, D.nw, n), dim3(B64), 0, st, t->dev.p, ws0);
+    if (D.ptt_lhs) {
+        hipLaunchKernelGGL(k64_grad<true>, dim3(D.nchg, D.nw, n), dim3(B64), 0, st, t->dev.p, ws0);
+        hipLaunchKernelGGL(k64_wg<true>, dim3(D.nchs, D.nw, n), dim3(B64), 0, st, t->dev.p, ws0);
+    } else {
+        hipLaunchKernelGGL(k64_gw, dim3(D.nchs, D.nw, n), dim3(B64), 0, st, t->dev.p, ws0);
+    }
     hipLaunchKernelGGL(k64_gpt, g_ploc(D, n), dim3(B64), 0, st, t->dev.p, ws0);
-    hipLaunchKernelGGL(k64_hxt<true>, g_node(D, n), dim3(B64), 0, st, t->dev.p, v, out, ws0);
+    launch_hxt<true>(t, st, v, out, ws0, n);
 }
 // z = FDPCG^-1 r and the partials of r . z into slot `slot`
 void enq_P(tomo64 *t, hipStream_t st, int ws0, int n, int slot) {
