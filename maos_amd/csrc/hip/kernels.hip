@@ -1149,7 +1149,7 @@ __global__ __launch_bounds__(256 * WS) void k_layer_m(KARGS, int psel_, int osel
         __syncthreads();
         if (threadIdx.x == 0 && part && si < ns)
             part[(long)(s0 + si) * partstride + by * PD.ltiles + bx] =
-                dadd(dadd(dadd(sh[0], sh[1], G.dot32), sh[2], G.dot32), sh[3], G.dot32);
+                dadd(dadd(sh[0], sh[1], G.dot32), dadd(sh[2], sh[3], G.dot32), G.dot32);
     }
 }
 
@@ -1163,9 +1163,9 @@ __global__ __launch_bounds__(256 * WS) void k_layer_m(KARGS, int psel_, int osel
 //
 // Layer tile sums: the order is the same whatever kernel takes the tile, so
 // that the tile shape, chosen by the number of systems, does not change a bit.
-// A 16 x 16 tile is four strips of 4 rows, added in order.  In a strip, two
-// adjacent columns are added first, then two adjacent rows, then these pairs of
-// rows (a thread's nodes here), then the 8 column pairs as a tree.
+// A 16 x 16 tile is four strips of 4 rows.  In a strip, two adjacent columns are
+// added first, then two adjacent rows, then these pairs of rows (a thread's
+// nodes here), then the 8 column pairs as a tree; the strips are added in pairs.
 template <bool LHS, typename RT, int CS, int LT, int WS = 1>
 __global__ __launch_bounds__(128 * WS) void k_layer_m8(KARGS, int psel_, int osel, int partsel) {
     KJOB;
@@ -1327,15 +1327,15 @@ __global__ __launch_bounds__(128 * WS) void k_layer_m8(KARGS, int psel_, int ose
             }
             dr[r] = dadd(d[0], d[1], G.dot32);
         }
-        // strips of 4 rows (the layer tile sums above), then 4 strips a tile:
+        // strips of 4 rows (the layer tile sums above), then the strips of a tile:
         // a wave holds LT / 2 rows, i.e. one 16 x 16 tile or two
         double d = dadd(dr[0], dr[1], G.dot32);
         if constexpr (R == 4) d = dadd(d, dadd(dr[2], dr[3], G.dot32), G.dot32);
         else d = dadd(d, __shfl_xor(d, 8, 64), G.dot32);
         for (int o : {1, 2, 4}) d = dadd(d, __shfl_xor(d, o, 64), G.dot32);
         constexpr int SL = 32 / R;  // lanes of a strip
-        double t = d;
-        for (int k = 1; k < 4; k++) t = dadd(t, __shfl_down(d, SL * k, 64), G.dot32);
+        double t = dadd(d, __shfl_down(d, SL, 64), G.dot32);
+        t = dadd(t, __shfl_down(t, 2 * SL, 64), G.dot32);
         const int lane = threadIdx.x & 63, half = (tid >> 6) * (LT / 32) + lane / (4 * SL);
         const int ty1 = (bx / ntx) * (LT / 16) + half;  // row of 16 x 16 tiles
         if (lane % (4 * SL) == 0 && active && part && si < ns && ty1 < (nyl + TILE - 1) / TILE)
