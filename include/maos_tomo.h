@@ -343,7 +343,7 @@ int  gpu_tomo_group_solve(gpu_tomo_group_t *grp, int mode, void *stream);
 /* Autotuner for a group: times whole graph solves of the group under the
  * column kernel (registers where a plan allows / LDS stages), the layer
  * tile rows (64 / 32 / 16) and the systems per workgroup of the WFS and layer
- * passes (1, 2, 4), by coordinate descent from the built-in heuristic, and
+ * passes (1, 2, 4), by coordinate descent from the built-in choice, and
  * sets the fastest on every member plan (as gpu_tomo_tune_set would, so a
  * plan's results alone and in the group stay the same bits).  choice[6]
  * (may be NULL) receives it in gpu_tomo_tune_set's order.  Overwrites the
@@ -420,7 +420,7 @@ int  gpu_tomo_autotune(gpu_tomo_t *g, int nsys, int *choice);
 
 /* Set the launch shape directly, e.g. to replay an autotuned choice without
  * timing: choice[6] = systems per workgroup of the WFS, layer and LDS
- * column kernels (each 1, 2 or 4, or 0 for the built-in heuristic), the
+ * column kernels (each 1, 2 or 4, or 0 for the built-in choice), the
  * layer tile rows (16, 32, 64, or 0 for the built-in choice), the column kernel
  * (1 registers where it applies, 2 LDS stages, 0 as 1; 2 also keeps the row
  * FFTs in LDS stages, which otherwise run in registers for single-plan
@@ -558,7 +558,8 @@ int  gpu_fit_solve(gpu_fit_t *g, int isys, const double *opdr, double *dmfit,
                    double *cgres);
 /* nsys <= nbatch systems with device buffers (FP32 layer vectors in, FP64
  * DM vectors out), enqueued on stream (0: the plan's own); no host sync.
- * Five launches per CG iteration, shared by the nsys systems.  d_dmfit
+ * Two launches per CG iteration (five where the operator is not assembled:
+ * directions far apart), shared by the nsys systems.  d_dmfit
  * holds the warm start when the plan has warm = 1. */
 int  gpu_fit_solve_dev(gpu_fit_t *g, const float *d_opdr, double *d_dmfit,
                        int nsys, void *stream);

@@ -12,9 +12,10 @@
 // 4k fitting-grid points per direction) and its CG is a chain of dependent
 // passes.  Each pass is one launch over the whole GPU, with work items
 // (point, direction, system) or (actuator, direction, system), so that a
-// thread does one short chain of dependent loads per pass; an iteration is
-// five launches (HA, W, HA' + low-rank terms, x/r update, p update) and a
-// batch of systems shares every launch.  Scalars (alpha, beta, the W1 and NW
+// thread does one short chain of dependent loads per pass, and a batch of
+// systems shares every launch.  An iteration is two launches with the assembled
+// operator (local boxes plus low rank, below) and five without it (HA, W, HA' +
+// low-rank terms, x/r update, p update).  Scalars (alpha, beta, the W1 and NW
 // projections) are fixed-order sums of per-workgroup partials, summed again
 // by every workgroup that needs them, so no launch waits on the host and a
 // system's bits do not depend on its batch neighbours.  (Running the whole
