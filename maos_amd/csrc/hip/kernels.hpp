@@ -18,16 +18,15 @@
 
 #include <cstdint>
 
+#include "launch_rules.hpp"
+
 namespace mtk {
 
 constexpr int MAXL = 16;      // layers
 constexpr int MAXW = 16;      // wavefront sensors (active)
 constexpr int MAXST = 8;      // FFT stages
-constexpr int TILE = 16;      // output tile edge of the WFS / layer passes
 constexpr int TAPS = 4;       // max ploc samples landing on one layer node per axis
 constexpr int ROWS = 16;      // rows per row-FFT workgroup (8 complex FFTs)
-constexpr int LTY = 64;       // tile height of the 16 x 64 layer kernel (k_layer_m8)
-constexpr int LTY2 = 32;      // of its 16 x 32 form
 constexpr int MAXN = 1024;    // largest FFT length (layer grid edge)
 
 // Matched-sampling ray of one (WFS, layer) pair: ploc index i maps to layer

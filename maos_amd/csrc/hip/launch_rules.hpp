@@ -1,0 +1,52 @@
+// Rules that choose the launch shape of a batch.  None of these choices
+// changes a result.  Host code without HIP.
+#pragma once
+#include <vector>
+
+namespace mtk {
+
+constexpr int TILE = 16;      // output tile edge of the WFS / layer passes
+constexpr int LTY = 64;       // tile height of the 16 x 64 layer kernel (k_layer_m8)
+constexpr int LTY2 = 32;      // tile height of the 16 x 32 layer kernel (k_layer_m8)
+
+// One job of a batch, as the layer pass sees it.
+struct LayerJob {
+    bool matched;       // matched rays; others take the generic kernel (TILE)
+    int tuned;          // chosen tile rows, 0: by the rule
+    bool fits2, fits;   // LTY2-row, LTY-row tiles fit every layer
+    long nodes;         // layer nodes of its systems
+};
+
+// Layer tile rows of each job.  Without a tuned choice: TILE rows, in the
+// split form where that applies, for a few small systems, LTY2 from about
+// 100 000 nodes in the launch on, whether they are one plan's systems or many
+// plans' (the kernel sees workgroups).  k_layer, us, 16 / 32 rows (64): 5184 nodes a
+// system, 1 system 4.8 5.4, 16: 5.7 6.3, 32: 7.0 6.2, 256: 25.9 15.1; 6272
+// nodes, 16: 6.2 5.6; 16 384 nodes, 1: 5.1 5.6, 8: 6.1 5.6, 64: 19.7 11.3; the
+// 30 m system, 1: 5.7 6.1 (12.4), 8: 11.4 8.5 (12.4), 32: 31.3 17.5 (19.3), 256:
+// 201 88 (91).  Jobs that stay on TILE rows (layers under LTY2 + 2 rows, a tuned
+// choice) are then a launch of their own, which has to be repaid: a group of
+// 8 small members (28-row layers) and 4 / 8 / 16 / 24 of 30 m, 10 iterations,
+// all on 16 rows against large ones on 32: 713 841 1051 1307 against 750 867 1020
+// 1248 us; 16 / 32 of 20 m: 647 889 against 688 892.
+constexpr long LTY2_NODES = 100000, LTY2_NODES_BESIDE = 600000;
+inline std::vector<int> layer_rows(const std::vector<LayerJob> &jobs) {
+    auto stays = [](const LayerJob &j) { return j.tuned == TILE || (!j.fits2 && j.tuned != LTY); };
+    long nodes = 0;      // of the LTY2 launch
+    bool beside = false;  // a TILE launch whatever the others do
+    for (const LayerJob &j : jobs) {
+        if (!j.matched) continue;
+        if (stays(j)) beside = true;
+        else if (j.tuned != LTY) nodes += j.nodes;
+    }
+    const int built_in = nodes >= (beside ? LTY2_NODES_BESIDE : LTY2_NODES) ? LTY2 : TILE;
+    std::vector<int> rows;
+    for (const LayerJob &j : jobs) {
+        if (!j.matched || stays(j)) rows.push_back(TILE);
+        else if (j.tuned == LTY) rows.push_back(j.fits ? LTY : TILE);
+        else rows.push_back(j.tuned ? j.tuned : built_in);
+    }
+    return rows;
+}
+
+}  // namespace mtk

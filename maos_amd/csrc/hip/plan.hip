@@ -451,21 +451,11 @@ void build_mreg(gpu_tomo *g, const std::vector<float2> &hM, const std::vector<in
     g->grp_blk_host = hgb;
 }
 
-// Layer tile rows for nsys systems of a plan (the shape does not change
-// results: p.Ap is summed per 16 x 16 nodes in one order).  Without a tuned
-// choice: TILE rows, in the split form where that applies, for a few small
-// systems, LTY2 from about 100 000 nodes in the launch on.  k_layer, us, 16 / 32
-// rows (64): 5184 nodes a system, 1 system 4.8 5.4, 16: 5.7 6.3, 32: 7.0 6.2,
-// 256: 25.9 15.1; 6272 nodes, 16: 6.2 5.6; 16 384 nodes, 1: 5.1 5.6, 8: 6.1
-// 5.6, 64: 19.7 11.3; the 30 m system, 1: 5.7 6.1 (12.4), 8: 11.4 8.5 (12.4),
-// 32: 31.3 17.5 (19.3), 256: 201 88 (91).
-constexpr long LTY2_NODES = 100000;
-int layer_rows(const gpu_tomo *g, int nsys) {
-    if (!g->G.matched || g->tune_lty == TILE) return TILE;
-    if (g->tune_lty == LTY) return g->lty_ok ? LTY : TILE;
-    if (!g->lty2_ok) return TILE;
-    return g->tune_lty == LTY2 || g->G.nxtot * nsys >= LTY2_NODES ? LTY2 : TILE;
+LayerJob layer_job(const gpu_tomo *g, int nsys) {
+    return LayerJob{g->G.matched != 0, g->tune_lty, g->lty2_ok, g->lty_ok, g->G.nxtot * nsys};
 }
+// Layer tile rows of a call on nsys systems of one plan.
+int layer_rows_alone(const gpu_tomo *g, int nsys) { return layer_rows({layer_job(g, nsys)})[0]; }
 
 void build_plan(gpu_tomo *g, const mt_recon_t *R) {
     if (!R || R->npsr <= 0 || R->npsr > MAXL || R->nwfs <= 0) fail(MT_EINVAL, "invalid recon (npsr/nwfs)");
@@ -1256,9 +1246,12 @@ std::unique_ptr<Batch> make_batch(const std::vector<gpu_tomo *> &plans, const st
                     sb.split = sb.matched && sb.pos == 1 && sb.cs == 1 && can_split(js) &&
                                wgs(js, [&](int j) { return (long)ptiles(j) * G(j).nwfs; }) <= SPLIT_WGS;
                 });
+    std::vector<LayerJob> lj;
+    for (size_t j = 0; j < b.hjob.size(); j++) lj.push_back(layer_job(b.plan[j], NS((int)j)));
+    const std::vector<int> lrows = layer_rows(lj);
     build_stage(b, b.layer,
                 [&](int j, std::vector<int> &k) {
-                    const int lty = layer_rows(b.plan[j], NS(j));
+                    const int lty = lrows[j];
                     k = {G(j).matched ? (lty == LTY ? 2 : lty == LTY2 ? 3 : 1) : 0};
                     return true;
                 },
@@ -2537,7 +2530,7 @@ int gpu_tomo_autotune(gpu_tomo_t *g, int nsys, int *choice) {
         // they fit) and systems per workgroup together
         {
             double best = 1e30;
-            int bestl = layer_rows(g, nsys), bestc = 1;
+            int bestl = layer_rows_alone(g, nsys), bestc = 1;
             for (int lty : {LTY, LTY2, TILE}) {
                 if (lty == LTY && !(g->G.matched && g->lty_ok)) continue;
                 if (lty == LTY2 && !(g->G.matched && g->lty2_ok)) continue;
@@ -2634,7 +2627,7 @@ int gpu_tomo_autotune(gpu_tomo_t *g, int nsys, int *choice) {
             choice[0] = g->tune_wfs;
             choice[1] = g->tune_layer;
             choice[2] = g->tune_col;
-            choice[3] = layer_rows(g, nsys);
+            choice[3] = layer_rows_alone(g, nsys);
             choice[4] = g->tune_colfft;
             choice[5] = g->tune_flights;
         }

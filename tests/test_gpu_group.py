@@ -115,3 +115,35 @@ def test_group_autotune_keeps_alone_bits(plans):
             for s in range(2):
                 assert np.array_equal(g.get_x(s)[0], alone[k][s]), "member %d slot %d (mode %d)" % (k, s, mode)
     grp.close()
+
+
+# members of groups at their default launch shape: layers on 16 x 32 tiles, the
+# same beside members whose layers are too small for them, all on 16 x 16
+L30, S8 = ("large30", configs.large30), ("b8", lambda: configs.batch_member(8.0, 4, 4))
+LARGE_GROUPS = {"all32": [L30] * 12, "beside": [L30] * 12 + [S8] * 4, "all16": [L30] * 4 + [S8] * 8}
+
+
+@pytest.mark.parametrize("name", list(LARGE_GROUPS))
+def test_large_default_groups_equal_alone(name):
+    """One system of each of 12 to 16 plans, the launch shape left to the
+    built-in rules: the bits of each plan solved alone."""
+    recon, plans = {}, []
+    for k, (key, mk) in enumerate(LARGE_GROUPS[name]):
+        cfg = mk()
+        if key not in recon:
+            recon[key] = tomo.Recon(cfg)
+        g = tomo.GpuTomo(recon[key], nbatch=1, maxit=4)
+        grad = workload.make_inputs(cfg, recon[key], 500 + k)
+        plans.append((g, grad, g.tomo(grad)[0]))
+    for g, grad, x1 in plans:
+        g.set_grad(0, grad)
+    grp = tomo.GpuGroup([(g, 0, 1) for g, grad, x1 in plans])
+    for mode in (0, 1):
+        grp.solve(mode=mode)
+        for k, (g, grad, x1) in enumerate(plans):
+            assert np.array_equal(g.get_x(0)[0], x1), "member %d (mode %d)" % (k, mode)
+    grp.close()
+    for g, grad, x1 in plans:
+        g.close()
+    for r in recon.values():
+        r.close()

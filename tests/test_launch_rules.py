@@ -1,0 +1,66 @@
+"""The rules that choose a batch's launch shape (launch_rules.hpp), compiled
+for the CPU."""
+import ctypes as C
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+SRC = r"""
+#include "launch_rules.hpp"
+using namespace mtk;
+extern "C" void layer_rows_of(int n, const long *j, int *rows) {  // j: matched, tuned, fits2, fits, nodes
+    std::vector<LayerJob> v;
+    for (int i = 0; i < n; i++, j += 5) v.push_back(LayerJob{j[0] != 0, (int)j[1], j[2] != 0, j[3] != 0, j[4]});
+    const std::vector<int> r = layer_rows(v);
+    for (int i = 0; i < n; i++) rows[i] = r[i];
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    d = tmp_path_factory.mktemp("rules")
+    (d / "rules.cpp").write_text(SRC)
+    so = str(d / "librules.so")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-shared", "-fPIC",
+                    "-I" + os.path.join(ROOT, "maos_amd", "csrc", "hip"), str(d / "rules.cpp"), "-o", so], check=True)
+    return C.CDLL(so)
+
+
+def rows_of(rules, jobs):
+    flat = [int(v) for j in jobs for v in j]
+    out = (C.c_int * len(jobs))()
+    rules.layer_rows_of(len(jobs), (C.c_long * len(flat))(*flat), out)
+    return list(out)
+
+
+def job(nodes, tuned=0, fits2=True, fits=True, matched=True):
+    return (matched, tuned, fits2, fits, nodes)
+
+
+L30, M20, S8 = 55296, 16384, 3136  # layer nodes of one 30 m, 20 m and 8 m system
+
+
+@pytest.mark.parametrize("jobs,rows", [
+    ([job(L30)], [16]),                                        # one system
+    ([job(2 * L30)], [32]),                                    # two of one plan
+    ([job(L30)] * 2, [32] * 2),                                # two plans of one each: the same launch
+    ([job(M20)] * 6, [16] * 6),                                # 98 304 nodes
+    ([job(M20)] * 7, [32] * 7),                                # 114 688
+    ([job(L30)] * 32, [32] * 32),
+    ([job(L30), job(L30, matched=False)], [16, 16]),           # the generic kernel's nodes are another launch's
+    ([job(L30, 16), job(12 * L30)], [16, 32]),                 # a tuned choice stays
+    ([job(L30, 16), job(L30)], [16, 16]),
+    ([job(L30, 32), job(L30)], [32, 32]),
+    ([job(L30, 64), job(L30, 64, fits=False)], [64, 16]),
+    ([job(M20, 32), job(S8, 32, fits2=False)], [32, 16]),
+    # members whose layers are too small for 32 rows need a launch of their
+    # own beside them, which large members have to repay
+    ([job(L30)] * 8 + [job(S8, fits2=False, fits=False)] * 8, [16] * 16),
+    ([job(L30)] * 16 + [job(S8, fits2=False, fits=False)] * 8, [32] * 16 + [16] * 8),
+])
+def test_layer_rows(rules, jobs, rows):
+    assert rows_of(rules, jobs) == rows
