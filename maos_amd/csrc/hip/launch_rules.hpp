@@ -1,6 +1,7 @@
 // Rules that choose the launch shape of a batch.  None of these choices
 // changes a result.  Host code without HIP.
 #pragma once
+#include <utility>
 #include <vector>
 
 namespace mtk {
@@ -47,6 +48,26 @@ inline std::vector<int> layer_rows(const std::vector<LayerJob> &jobs) {
         else rows.push_back(j.tuned ? j.tuned : built_in);
     }
     return rows;
+}
+
+inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
+
+// Systems per workgroup: the most of cmax, cmax/2, .., 1 that keeps >= thresh
+// workgroups in the launch (thresh4 for 4 systems) and leaves at most a fifth
+// of their slots empty; jw = (workgroups per system, systems) per job.  The
+// kernels compute an empty slot like a filled one and drop it: groups of 8 / 16
+// / 32 one-system 30 m members, 10 iterations, with 2, 2, 4 slots (as the number
+// of workgroups alone would have it) 471 718 1143 us, with one 450 583 915.
+inline int pick_cs(const std::vector<std::pair<long, int>> &jw, int cmax, int thresh, int thresh4) {
+    for (int cs = cmax; cs > 1; cs >>= 1) {
+        long tot = 0, filled = 0;
+        for (auto &p : jw) {
+            tot += p.first * ceil_div(p.second, cs);
+            filled += p.first * p.second;
+        }
+        if (tot >= (cs == 4 ? thresh4 : thresh) && 5 * filled >= 4 * cs * tot) return cs;
+    }
+    return 1;
 }
 
 }  // namespace mtk

@@ -1115,18 +1115,6 @@ void build_stage(Batch &B, Stage &out, KeyF key, GridF grid, SubF fill,
         out.push_back(std::move(sub));
     }
 }
-int ceil_div(int a, int b) { return (a + b - 1) / b; }
-// Systems per workgroup: the most of cmax, cmax/2, .., 1 that keeps >= thresh
-// workgroups in the launch (thresh4 for 4 systems); jw = (workgroups per
-// system, systems) per job.
-int pick_cs(const std::vector<std::pair<long, int>> &jw, int cmax, int thresh, int thresh4) {
-    for (int cs = cmax; cs > 1; cs >>= 1) {
-        long tot = 0;
-        for (auto &p : jw) tot += p.first * ceil_div(p.second, cs);
-        if (tot >= (cs == 4 ? thresh4 : thresh)) return cs;
-    }
-    return 1;
-}
 
 // Launches of at most this many workgroups (one per CU) take the split forms
 // of k_wfs_m (tomo.pos = 1) and the layer kernels.  us per launch, back to back,

@@ -17,6 +17,11 @@ extern "C" void layer_rows_of(int n, const long *j, int *rows) {  // j: matched,
     const std::vector<int> r = layer_rows(v);
     for (int i = 0; i < n; i++) rows[i] = r[i];
 }
+extern "C" int pick_cs_of(int n, const long *wg, const int *ns, int cmax, int thresh, int thresh4) {
+    std::vector<std::pair<long, int>> v;
+    for (int i = 0; i < n; i++) v.push_back({wg[i], ns[i]});
+    return pick_cs(v, cmax, thresh, thresh4);
+}
 """
 
 
@@ -64,3 +69,27 @@ L30, M20, S8 = 55296, 16384, 3136  # layer nodes of one 30 m, 20 m and 8 m syste
 ])
 def test_layer_rows(rules, jobs, rows):
     assert rows_of(rules, jobs) == rows
+
+
+@pytest.mark.parametrize("jw,cmax,cs", [
+    # (workgroups per system, systems) per job; 512 workgroups for 2, 1100 for 4
+    ([(96, 1)], 4, 1),
+    ([(96, 10)], 4, 1),
+    ([(96, 11)], 4, 2),
+    ([(96, 45)], 4, 4),
+    ([(96, 45)], 2, 2),
+    ([(36, 29)], 4, 2),
+    # jobs of one system fill one slot however many there are
+    ([(96, 1)] * 6, 4, 1),
+    ([(96, 1)] * 32, 4, 1),
+    ([(96, 2)] * 16, 4, 2),
+    ([(96, 3)] * 16, 4, 1),
+    ([(96, 4)] * 16, 4, 4),
+    # a few of them beside a large job leave its choice
+    ([(96, 48), (36, 1)], 4, 4),
+    ([(96, 4)] + [(96, 1)] * 20, 4, 1),
+])
+def test_systems_per_workgroup(rules, jw, cmax, cs):
+    wg = (C.c_long * len(jw))(*[w for w, _ in jw])
+    ns = (C.c_int * len(jw))(*[n for _, n in jw])
+    assert rules.pick_cs_of(len(jw), wg, ns, cmax, 512, 1100) == cs
