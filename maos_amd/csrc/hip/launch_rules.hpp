@@ -1,6 +1,7 @@
 // Rules that choose the launch shape of a batch.  None of these choices
 // changes a result.  Host code without HIP.
 #pragma once
+#include <algorithm>
 #include <utility>
 #include <vector>
 
@@ -68,6 +69,38 @@ inline int pick_cs(const std::vector<std::pair<long, int>> &jw, int cmax, int th
         if (tot >= (cs == 4 ? thresh4 : thresh) && 5 * filled >= 4 * cs * tot) return cs;
     }
     return 1;
+}
+
+// The group autotuner's search: coordinate descent from the built-in choice
+// over the column kernel, the layer tile rows, then the systems per workgroup
+// of the WFS and layer passes; a change is kept when it saves more than 2 %.
+// timed: the time of a choice, in gpu_tomo_tune_set's order.  A tile shape that
+// fits no member (fits2, fits: LTY2, LTY rows fit one) would be TILE rows again.
+template <typename Timed> void group_descent(bool fits2, bool fits, Timed timed, int *best) {
+    const int start[6] = {0, 0, 0, 0, 0, 1};
+    std::copy(start, start + 6, best);
+    double tbest = timed((const int *)best);
+    auto trial = [&](int k, const std::vector<int> &vals) {
+        for (int v : vals) {
+            if (v == best[k]) continue;
+            int c[6];
+            std::copy(best, best + 6, c);
+            c[k] = v;
+            const double t = timed((const int *)c);
+            if (t < tbest * 0.98) {
+                tbest = t;
+                best[k] = v;
+            }
+        }
+    };
+    trial(4, {2});
+    std::vector<int> rows;
+    if (fits) rows.push_back(LTY);
+    if (fits2) rows.push_back(LTY2);
+    rows.push_back(TILE);
+    trial(3, rows);
+    trial(0, {1, 2, 4});
+    trial(1, {1, 2, 4});
 }
 
 }  // namespace mtk

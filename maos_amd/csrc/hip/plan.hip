@@ -2420,28 +2420,13 @@ int gpu_tomo_group_autotune(gpu_tomo_group_t *grp, int *choice) {
             std::sort(ts.begin(), ts.end());
             return (double)ts[ts.size() / 2];
         };
-        // coordinate descent from the heuristic: column kernel, layer tile
-        // rows, then systems per workgroup of the WFS and layer passes; a
-        // change is kept when it saves more than 2 %
-        int best[6] = {0, 0, 0, 0, 0, 1};
-        double tbest = timed(best);
-        auto trial = [&](int k, std::initializer_list<int> vals) {
-            for (int v : vals) {
-                if (v == best[k]) continue;
-                int c[6];
-                std::copy(best, best + 6, c);
-                c[k] = v;
-                const double t = timed(c);
-                if (t < tbest * 0.98) {
-                    tbest = t;
-                    best[k] = v;
-                }
-            }
-        };
-        trial(4, {2});
-        trial(3, {LTY2, TILE});
-        trial(0, {1, 2, 4});
-        trial(1, {1, 2, 4});
+        bool fits = false, fits2 = false;
+        for (const gpu_tomo *g : grp->plans) {
+            fits |= g->lty_ok;
+            fits2 |= g->lty2_ok;
+        }
+        int best[6];
+        group_descent(fits2, fits, timed, best);
         (void)hipEventDestroy(e0);
         (void)hipEventDestroy(e1);
         group_apply(grp, best);

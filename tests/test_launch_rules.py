@@ -22,6 +22,9 @@ extern "C" int pick_cs_of(int n, const long *wg, const int *ns, int cmax, int th
     for (int i = 0; i < n; i++) v.push_back({wg[i], ns[i]});
     return pick_cs(v, cmax, thresh, thresh4);
 }
+extern "C" void descent_of(int fits2, int fits, double (*timed)(const int *), int *best) {
+    group_descent(fits2 != 0, fits != 0, timed, best);
+}
 """
 
 
@@ -93,3 +96,23 @@ def test_systems_per_workgroup(rules, jw, cmax, cs):
     wg = (C.c_long * len(jw))(*[w for w, _ in jw])
     ns = (C.c_int * len(jw))(*[n for _, n in jw])
     assert rules.pick_cs_of(len(jw), wg, ns, cmax, 512, 1100) == cs
+
+
+@pytest.mark.parametrize("fits2,fits", [(1, 1), (1, 0), (0, 0)])
+@pytest.mark.parametrize("rows", [0, 16, 32, 64])
+@pytest.mark.parametrize("col", [0, 2])
+def test_group_descent_finds_the_fastest(rules, rows, col, fits2, fits):
+    """The search times every layer tile shape that fits and both column
+    kernels, and keeps the fastest (0: the built-in choice)."""
+    tried = []
+
+    def timed(c):
+        tried.append(list(c[:6]))
+        return 1.0 + 0.1 * (c[3] != rows) + 0.1 * (c[4] != col) + 0.1 * (c[0] != 2) + 0.01 * (c[1] != 1)
+
+    best = (C.c_int * 6)()
+    rules.descent_of(fits2, fits, C.CFUNCTYPE(C.c_double, C.POINTER(C.c_int))(timed), best)
+    shapes = {0, 16} | ({32} if fits2 else set()) | ({64} if fits else set())
+    assert tried[0] == [0, 0, 0, 0, 0, 1]
+    assert {t[3] for t in tried} == shapes
+    assert list(best) == [2, 0, 0, rows if rows in shapes else 0, col, 1]
