@@ -33,6 +33,7 @@
 #include "fit_internal.hpp"
 #include "rays.hpp"
 #include "solve64.hpp"
+#include "staging.hpp"
 #include "kernels.hpp"
 #include "launch.hpp"
 #include "maos_tomo.h"
@@ -150,13 +151,15 @@ struct ProfEv {
     hipEvent_t a, b;
 };
 
-// Pinned host staging of a plan's own host calls.
-struct PinBuf {
-    float *p = nullptr;
-    void alloc(size_t n) { HIPCHK(hipHostMalloc((void **)&p, sizeof(float) * n, hipHostMallocDefault)); }
-    ~PinBuf() {
-        if (p) (void)hipHostFree(p);
+// Pinned host memory for a plan's staging (staging.hpp).
+struct HipPinned {
+    static void *get(size_t bytes) {
+        void *p = nullptr;
+        if (hipHostMalloc(&p, bytes, hipHostMallocDefault) == hipSuccess) return p;
+        (void)hipGetLastError();  // the refusal is not the next call's error
+        return nullptr;
     }
+    static void put(void *p) { (void)hipHostFree(p); }
 };
 
 struct gpu_tomo {
@@ -199,7 +202,7 @@ struct gpu_tomo {
     DevBuf<double> part_pap, part_rz, part_rr, part_bb, rz, alpha, res;
     DevBuf<int> stop;
     // host staging
-    PinBuf pin;                 // one system's gradients, or its residual and solution
+    Staging<HipPinned> pin;     // one system's gradients, or its residual and solution
     std::vector<float> hstage;
     // graph
     hipGraph_t graph = nullptr;
@@ -1575,10 +1578,11 @@ void pack_grad(const gpu_tomo *g, const double *grad, float *dst) {
         }
     }
 }
-// Host gradients into slot isys, through the plan's pinned staging (a copy
+// Host gradients into slot isys, through the plan's staging (pinned: a copy
 // from pageable memory stages and waits inside the runtime; 8 loops of a group,
 // gradients in and solutions out: 1354 -> 1205 us a step; one 30 m solve: 930
-// -> 880).  wait: the copy has completed on return (without it the staging must
+// -> 880.  About 220 KB a plan of the 30 m system, taken at set-up so that a
+// first call is no slower).  wait: the copy has completed on return (without it the staging must
 // not be written before the stream is waited for).
 void to_dev_grad(gpu_tomo *g, int isys, const double *grad, bool wait = true) {
     const Geom &G = g->G;
