@@ -171,19 +171,27 @@ __device__ double reduce_partials(const double *part, int n, double *sh, int f32
     }
     return block_sum(f32 ? (double)vf : v, sh, f32);
 }
-// Product / fused accumulation of a dot-product term, in FP32 for mode 3.
+// Product / sum / fused accumulation of dot-product terms, in FP32 for mode 3.
 __device__ __forceinline__ double dmul(double a, double b, int f32) {
     return f32 ? (double)((float)a * (float)b) : a * b;
 }
 __device__ __forceinline__ double dadd(double a, double b, int f32) {
+#pragma clang fp contract(off)
     return f32 ? (double)((float)a + (float)b) : a + b;
 }
 __device__ __forceinline__ double dfma(double a, double b, double c, int f32) {
     return f32 ? (double)fmaf((float)a, (float)b, (float)c) : a * b + c;
 }
-// wa a + wb b with the rounding fixed (the compiler picks which product to fuse
-// from its surroundings): the layer kernels agree bit for bit.
+// The forms of the matched WFS and layer kernels agree bit for bit, whichever a
+// launch takes, so the roundings of their terms are fixed here (left to itself
+// the compiler picks what to fuse from its surroundings; dadd never takes a
+// product in).  wa a + wb b:
 template <typename T> __device__ __forceinline__ T lerp2(T wa, T a, T wb, T b) { return fma(wa, a, wb * b); }
+// a + l2c (20 c - 8 s4 + 2 sd + s2), the regulariser at a node (the products by
+// powers of two are exact):
+template <typename T> __device__ __forceinline__ T l2_node(T a, T l2c, T c, T s4, T sd, T s2) {
+    return fma(l2c, fma(T(2), sd, fma(T(20), c, T(-8) * s4)) + s2, a);
+}
 __device__ __forceinline__ double ddiv(double a, double b, int f32) {
     return f32 ? (double)((float)a / (float)b) : a / b;
 }
@@ -880,7 +888,7 @@ __global__ __launch_bounds__(256 * WS) void k_wfs_m(KARGS, int xsel) {
             // otherwise load those used only past a branch separately)
             asm volatile("" ::"s"(m.wx), "s"(m.wy), "s"(nyl), "s"(xo));
             const float *xl = xs + xo;
-            const RT fx = m.fx, fy = m.fy;
+            const RT fx = m.fx, fy = m.fy, gx = RT(1) - fx, gy = RT(1) - fy;
             const bool fast = tx0 - POS >= m.ax0 && tx0 + TILE + POS <= (m.wx ? m.ax1 - 1 : m.ax1) &&
                               ty0 - POS >= m.ay0 && ty0 + TILE + POS <= (m.wy ? m.ay1 - 1 : m.ay1);
             // systems past ns read system ns-1 (in range; never stored)
@@ -891,13 +899,14 @@ __global__ __launch_bounds__(256 * WS) void k_wfs_m(KARGS, int xsel) {
                     const float *t = xl + (long)min(si, ns - 1) * G.nxtot + o;
                     RT h[3];
 #pragma unroll
-                    for (int k = 0; k < 3; k++) h[k] = (RT(1) - fx) * (RT)t[k * nxl] + fx * (RT)t[k * nxl + 1];
+                    for (int k = 0; k < 3; k++) h[k] = lerp2(gx, (RT)t[k * nxl], fx, (RT)t[k * nxl + 1]);
+                    const RT v0 = lerp2(gy, h[0], fy, h[1]), v1 = lerp2(gy, h[1], fy, h[2]);
                     if constexpr (WS > 1) {
-                        v[0][si] = (RT(1) - fy) * h[0] + fy * h[1];
-                        v[1][si] = (RT(1) - fy) * h[1] + fy * h[2];
+                        v[0][si] = v0;
+                        v[1][si] = v1;
                     } else {
-                        v[0][si] += (RT(1) - fy) * h[0] + fy * h[1];
-                        v[1][si] += (RT(1) - fy) * h[1] + fy * h[2];
+                        v[0][si] += v0;
+                        v[1][si] += v1;
                     }
                 }
             } else {
@@ -914,7 +923,7 @@ __global__ __launch_bounds__(256 * WS) void k_wfs_m(KARGS, int xsel) {
                     for (int si = 0; si < CS; si++) {
                         const float *t = xl + (long)min(si, ns - 1) * G.nxtot;
                         const RT a = t[o00], b = t[o10], c = t[o01], d = t[o11];
-                        const RT h = (RT(1) - fy) * ((RT(1) - fx) * a + fx * b) + fy * ((RT(1) - fx) * c + fx * d);
+                        const RT h = lerp2(gy, lerp2(gx, a, fx, b), fy, lerp2(gx, c, fx, d));
                         if constexpr (WS > 1) v[r][si] = ok ? h : RT(0);
                         else v[r][si] += ok ? h : RT(0);
                     }
@@ -960,11 +969,11 @@ __global__ __launch_bounds__(256 * WS) void k_wfs_m(KARGS, int xsel) {
 #pragma unroll
                         for (int zx = 0; zx < NP; zx++) {
                             const RT o = opd[si][(b + zy) * H + a + zx];
-                            gx += (RT)c[zy * NP + zx].x * o;
-                            gy += (RT)c[zy * NP + zx].y * o;
+                            gx = fma((RT)c[zy * NP + zx].x, o, gx);
+                            gy = fma((RT)c[zy * NP + zx].y, o, gy);
                         }
-                    wgx[si][i] = (RT)ne.x * gx + (RT)ne.z * gy;
-                    wgy[si][i] = (RT)ne.z * gx + (RT)ne.y * gy;
+                    wgx[si][i] = lerp2((RT)ne.x, gx, (RT)ne.z, gy);
+                    wgy[si][i] = lerp2((RT)ne.z, gx, (RT)ne.y, gy);
                 }
             }
         }
@@ -989,7 +998,7 @@ __global__ __launch_bounds__(256 * WS) void k_wfs_m(KARGS, int xsel) {
             if (si < ns) {
                 RT acc = 0;
 #pragma unroll
-                for (int z = 0; z < NP2; z++) acc += (RT)c[z].x * wgx[si][sidx[z]] + (RT)c[z].y * wgy[si][sidx[z]];
+                for (int z = 0; z < NP2; z++) acc += lerp2((RT)c[z].x, wgx[si][sidx[z]], (RT)c[z].y, wgy[si][sidx[z]]);
                 q[((long)(s0 + si) * G.nwfs + w) * G.nploc + py * pnx + px] = acc;
             }
         }
@@ -1132,7 +1141,7 @@ __global__ __launch_bounds__(256 * WS) void k_layer_m(KARGS, int psel_, int osel
                 const RT s4 = P(-1, 0) + P(1, 0) + P(0, -1) + P(0, 1);
                 const RT sd = P(-1, -1) + P(1, -1) + P(-1, 1) + P(1, 1);
                 const RT s2 = P(-2, 0) + P(2, 0) + P(0, -2) + P(0, 2);
-                a += (RT)G.l2c[l] * (RT(20) * c - RT(8) * s4 + RT(2) * sd + s2);
+                a = l2_node(a, (RT)G.l2c[l], c, s4, sd, s2);
                 dot[si] = dmul(c, a, G.dot32);
             } else {
                 dot[si] = dmul(a, a, G.dot32);
@@ -1317,7 +1326,7 @@ __global__ __launch_bounds__(128 * WS) void k_layer_m8(KARGS, int psel_, int ose
                         const RT s4 = P(-1, 0) + P(1, 0) + P(0, -1) + P(0, 1);
                         const RT sd = P(-1, -1) + P(1, -1) + P(-1, 1) + P(1, 1);
                         const RT s2 = P(-2, 0) + P(2, 0) + P(0, -2) + P(0, 2);
-                        a += (RT)G.l2c[l] * (RT(20) * cv - RT(8) * s4 + RT(2) * sd + s2);
+                        a = l2_node(a, (RT)G.l2c[l], cv, s4, sd, s2);
                         d[c] = dmul(cv, a, G.dot32);
                     } else {
                         d[c] = dmul(a, a, G.dot32);

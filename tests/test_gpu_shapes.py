@@ -21,7 +21,7 @@ CFGS = {
 }
 
 
-@pytest.mark.parametrize("mode", [0, 1, 3])
+@pytest.mark.parametrize("mode", [0, 1, 2, 3])
 @pytest.mark.parametrize("name", list(CFGS))
 def test_tile_rows_and_split_bit_exact(name, mode):
     """Twelve systems in one call (above the split form's bound on all but the
