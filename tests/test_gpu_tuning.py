@@ -16,14 +16,14 @@ def _batch(r, cfg, n):
     return np.stack([workload.make_inputs(cfg, r, 40 + s) for s in range(n)])
 
 
-@pytest.mark.parametrize("rows", [0, 32])
+@pytest.mark.parametrize("rows", [0, 32, 64])
 @pytest.mark.parametrize("colk", [1, 2])
 @pytest.mark.parametrize("mode", [0, 1, 3])
 def test_systems_per_workgroup_bit_exact(large30, mode, colk, rows):
     """Five systems (one partial workgroup for every choice above 1) solved
     under each systems-per-workgroup choice and by the heuristic, with the
     register column kernel (1, which has no such choice) and the LDS column
-    kernel (2), on 16 x 64 (0: the default) and 16 x 32 layer tiles:
+    kernel (2), on 16 x 64 and 16 x 32 layer tiles and the built-in choice (0):
     identical solutions and residuals."""
     cfg, r = large30
     grads = _batch(r, cfg, 5)
