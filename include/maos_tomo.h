@@ -568,6 +568,9 @@ int  gpu_fit_solve_dev(gpu_fit_t *g, const float *d_opdr, double *d_dmfit,
  *   L : out = beta * out + alpha * FitL a (cufit_grid::L) */
 int  gpu_fit_R(gpu_fit_t *g, const double *opdr, double *out, double alpha);
 int  gpu_fit_L(gpu_fit_t *g, const double *a, double *out, double alpha, double beta);
+/* Plan facts: FitL assembled (1) or in matrix-free passes (0); the most box
+ * entries of a row (0 in matrix-free passes) and the low-rank columns. */
+int  gpu_fit_info(const gpu_fit_t *g, int *assembled, int *entries, int *lowrank);
 /* Residuals of the last solve. */
 int  gpu_fit_residuals(gpu_fit_t *g, double *cgres, int nsys);
 /* MVM assembly: columns [col0, col0 + ncol) of the control matrix

@@ -168,6 +168,7 @@ def lib():
     L.gpu_fit_solve_dev.argtypes = [vp, vp, vp, C.c_int, vp]
     L.gpu_fit_R.argtypes = [vp, dp, dp, C.c_double]
     L.gpu_fit_L.argtypes = [vp, dp, dp, C.c_double, C.c_double]
+    L.gpu_fit_info.argtypes = [vp, ip, ip, ip]
     L.gpu_fit_residuals.argtypes = [vp, dp, C.c_int]
     L.gpu_mvm_assemble.argtypes = [vp, vp, C.c_long, C.c_long, dp]
     L.gpu_fit_free.argtypes = [vp]
@@ -222,7 +223,7 @@ EXPORTS = [
     "gpu_tomo_server_usage", "gpu_tomo_server_autotune", "gpu_tomo_server_update_cn2", "gpu_tomo_server_free", "gpu_tomo_autotune", "gpu_tomo_tune_set", "gpu_tomo_info", "gpu_tomo_residuals", "gpu_tomo_L", "gpu_tomo_R", "gpu_tomo_P",
     "gpu_tomo_sizes", "gpu_tomo_profile", "gpu_tomo_profile_read", "gpu_tomo_precision",
     "mt_fit_create", "mt_fit_recon", "mt_fit_sizes", "mt_fit_free", "gpu_fit_setup", "gpu_fit_solve",
-    "gpu_fit_solve_dev", "gpu_fit_R", "gpu_fit_L", "gpu_fit_residuals", "gpu_fit_free", "gpu_mvm_assemble",
+    "gpu_fit_solve_dev", "gpu_fit_R", "gpu_fit_L", "gpu_fit_info", "gpu_fit_residuals", "gpu_fit_free", "gpu_mvm_assemble",
     "mt_conf_new", "mt_conf_free", "mt_conf_add_path", "mt_conf_read", "mt_conf_has", "mt_conf_str",
     "mt_conf_strarr", "mt_conf_dbl", "mt_conf_unused",
     "mt_bin_read", "mt_bin_write", "mt_bin_free", "mt_bin_info", "mt_bin_data", "mt_bin_child",

@@ -1651,6 +1651,15 @@ int gpu_fit_L(gpu_fit_t *g, const double *a, double *out, double alpha, double b
     });
 }
 
+int gpu_fit_info(const gpu_fit_t *g, int *assembled, int *entries, int *lowrank) {
+    if (!g) return MT_EINVAL;
+    const FitDev &D = g->H;
+    if (assembled) *assembled = D.asm_ok;
+    if (entries) *entries = D.asm_ok ? *std::max_element(D.etot, D.etot + D.ndm) : 0;
+    if (lowrank) *lowrank = D.nlr;
+    return MT_OK;
+}
+
 int gpu_fit_residuals(gpu_fit_t *g, double *cgres, int nsys) {
     if (!g || !cgres || nsys <= 0 || nsys > g->nbatch) return MT_EINVAL;
     return fguarded([&] {

@@ -517,6 +517,12 @@ class GpuFit:
         except Exception:
             pass
 
+    def info(self):
+        """gpu_fit_info: dict(assembled, entries, lowrank)."""
+        v = [C.c_int() for _ in range(3)]
+        _abi.check(_abi.lib().gpu_fit_info(self._h, *[C.byref(a) for a in v]), "gpu_fit_info")
+        return dict(zip(("assembled", "entries", "lowrank"), [a.value for a in v]))
+
     def solve(self, opdr, isys=0):
         """curecon_t::fit: (dmfit, cgres, status) from tomography layers."""
         x = np.ascontiguousarray(opdr, dtype=np.float64)

@@ -231,32 +231,53 @@ def test_fit_graph_cache_eviction_in_flight(fitsys):
 
 
 # name: (aperture, directions' ring radius in arcsec, DM spacings, direction
-# heights, systems); sizes at the edges of the apply's tiles (16 x 4
-# actuators, 20 register entries a wave, 16 systems a workgroup)
-ASSEMBLED = {
-    "one_dm": (6.0, 0.0, [0.5], float("inf"), 1),            # box within the registers, partial tiles
-    "spacings": (8.0, 10.0, [0.5, 0.45], float("inf"), 5),   # spacings differ: hull of the rows' boxes
-    "wide": (12.0, 30.0, [0.5, 0.5], float("inf"), 3),       # boxes past the registers
-    "finite": (12.0, 10.0, [0.5, 0.5], 90e3, 18),            # converging directions, more systems than a workgroup holds
-    "matrix_free": (10.0, 120.0, [0.5, 0.5], float("inf"), 3),  # boxes too large: the five-pass form
+# heights, systems, assembled, bounds of the entries of a row); sizes at the
+# edges of the apply's tiles (16 x 4 actuators, 20 register entries in each of
+# four waves, 16 systems a workgroup)
+INF = float("inf")
+FORMS = {
+    "one_dm": (6.0, 0.0, [0.5], INF, 1, 1, (1, 80)),              # box within the registers, partial tiles
+    "spacings": (8.0, 10.0, [0.5, 0.45], INF, 5, 1, (81, 256)),   # spacings differ: hull of the rows' boxes
+    "wide": (12.0, 30.0, [0.5, 0.5], INF, 3, 1, (81, 256)),       # boxes past the registers
+    "finite": (12.0, 10.0, [0.5, 0.5], 90e3, 18, 1, (1, 256)),    # converging directions, more systems than a workgroup holds
+    "matrix_free": (10.0, 120.0, [0.5, 0.5], INF, 3, 0, (0, 0)),  # boxes too large: the five-pass form
 }
 
 
-@pytest.mark.parametrize("name", list(ASSEMBLED))
+def form_plan(name):
+    """(Recon, plan maker) of a form: plan maker(n, maxit) -> (FitSetup, GpuFit)."""
+    D, ring, dxs, hs = FORMS[name][:4]
+    base = configs.batch_member(D, 2, 2)
+    th = [(0.0, 0.0, 0.5)] + [(ring * np.cos(t), ring * np.sin(t), 0.125) for t in (0.3, 1.9, 3.2, 5.0)]
+    dms = [dict(ht=11800.0 * k, dx=dx, offset=0.5 * k, guard=1.0, iac=0.0) for k, dx in enumerate(dxs)]
+
+    def conf(maxit, warm=0):
+        return configs.fit_for(base, dm=dms, fit=th, fit_hs=[hs] * len(th), fit_maxit=maxit, warm=warm)
+
+    r = tomo.Recon(configs.with_fit_dirs(base, conf(1)))
+
+    def make(n, maxit, warm=0):
+        f = tomo.FitSetup(r, conf(maxit, warm))
+        assert f.rec.maxit == maxit
+        g = tomo.GpuFit(r, f, nbatch=n)
+        print("case", name, "nact", f.nact, "nfloc", f.nfloc, g.info(), flush=True)
+        return f, g
+
+    return r, make
+
+
+@pytest.mark.parametrize("name", list(FORMS))
 def test_fit_operator_forms(name):
     """FitL and the solve of every geometry the assembled operator accepts,
     and of one it leaves to the matrix-free passes, against the oracle; a
     system's result is the same bits in every batch.  L: two FP64 orders of
     the same sums, under 1e3 terms of 1e-16 each (1e-12)."""
-    D, ring, dxs, hs, n = ASSEMBLED[name]
-    base = configs.batch_member(D, 2, 2)
-    th = [(0.0, 0.0, 0.5)] + [(ring * np.cos(t), ring * np.sin(t), 0.125) for t in (0.3, 1.9, 3.2, 5.0)]
-    dms = [dict(ht=11800.0 * k, dx=dx, offset=0.5 * k, guard=1.0, iac=0.0) for k, dx in enumerate(dxs)]
-    fc = configs.fit_for(base, dm=dms, fit=th, fit_hs=[hs] * len(th), fit_maxit=12)
-    r = tomo.Recon(configs.with_fit_dirs(base, fc))
-    f = tomo.FitSetup(r, fc)
-    print("case", name, "nact", f.nact, "nfloc", f.nfloc, flush=True)
-    g, o = tomo.GpuFit(r, f, nbatch=n), FitOracle(r, f, nthread=8)
+    n, assembled, (lo, hi) = FORMS[name][4:]
+    r, make = form_plan(name)
+    f, g = make(n, 12)
+    i = g.info()
+    assert i["assembled"] == assembled and lo <= i["entries"] <= hi
+    o = FitOracle(r, f, nthread=8)
     rng = np.random.default_rng(7)
     a = rng.standard_normal(f.nact)
     assert rel(g.L(a), o.fit_l(a)) < 1e-12
@@ -271,3 +292,49 @@ def test_fit_operator_forms(name):
     g.close()
     dx.free()
     da.free()
+
+
+@pytest.mark.parametrize("more", [1, 4])
+@pytest.mark.parametrize("name", ["spacings", "finite", "matrix_free"])
+def test_fit_restart_past_100(name, more):
+    """The restart at iteration 100 forms r = b - A x and starts over from it,
+    so a cold solve of 100 + m iterations is the cold solve of 100 followed by m
+    from its commands: a warm solve of the same plan form, and the oracle's.
+    (The whole solve is chaotic in FP64 and bounds nothing here.  m steps are not:
+    these differ by the order of their sums, some 1e3 terms of 1e-16 each in r,
+    which carries the step; 1e-9 as for the short solves above.)  A system's bits
+    are the same alone and in the batch."""
+    n = 3
+    r, make = form_plan(name)
+    xs = (np.random.default_rng(8).standard_normal((n, r.nx)) * 1e-7).astype(np.float32)
+    dx = DevArray.of(xs)
+
+    def cold(maxit):
+        f, g = make(n, maxit)
+        assert g.info()["assembled"] == FORMS[name][5]
+        da = DevArray((n, f.nact), np.float64)
+        g.solve_dev(dx.ptr, da.ptr, nsys=n)
+        sync()
+        return g, da, da.numpy(), g.residuals(n)
+
+    g, d100, a100, _ = cold(100)
+    g.close()
+    g, da, a, res = cold(100 + more)
+    f, w = make(n, more, warm=1)
+    w.solve_dev(dx.ptr, d100.ptr, nsys=n)  # from the commands of the 100
+    sync()
+    aw, resw = d100.numpy(), w.residuals(n)
+    for k in range(n):
+        a1, res1, _ = g.solve(xs[k].astype(np.float64), isys=k)
+        assert np.array_equal(a1, a[k]) and res1 == res[k], k
+    ao, reso = FitOracle(r, f, nthread=8).solve(xs[0].astype(np.float64), more, a0=a100[0])
+    print("%s +%d: to warm %.2e, to oracle %.2e, step %.2e; residual %.9e warm %.9e oracle %.9e"
+          % (name, more, rel(a[0], aw[0]), rel(a[0], ao), rel(a[0], a100[0]), res[0], resw[0], reso), flush=True)
+    assert rel(a[0], a100[0]) > 1e-6  # the steps after the restart show at this tolerance
+    for k in range(n):
+        assert rel(a[k], aw[k]) < 1e-9 and abs(res[k] - resw[k]) <= 1e-6 * res[k], k
+    assert rel(a[0], ao) < 1e-9 and abs(res[0] - reso) <= 1e-6 * reso
+    g.close()
+    w.close()
+    for d in (dx, da, d100):
+        d.free()
