@@ -338,3 +338,72 @@ def test_fit_restart_past_100(name, more):
     w.close()
     for d in (dx, da, d100):
         d.free()
+
+
+def fit_l_80(recon, fit):
+    """FitL in extended precision (numpy's 80-bit long double) from the set-up's
+    own 64-bit taps and weights."""
+    f, LD = fit.rec, np.longdouble
+    px, py = f.fox + np.arange(f.fnx) * f.fdx, f.foy + np.arange(f.fny) * f.fdx
+
+    def axis(u, n):
+        m, i = np.zeros((len(u), n), LD), np.floor(u).astype(int)
+        for k, w in ((i, 1 - (u - i)), (i + 1, u - i)):
+            ok = (k >= 0) & (k < n) & (w > 1e-15)
+            m[np.nonzero(ok)[0], k[ok]] = w[ok]
+        return m
+
+    dms, off = fit.grids(), [0]
+    for d in dms:
+        off.append(off[-1] + d["nx"] * d["ny"])
+    ha = []
+    for i in range(f.nfit):
+        sc = [1.0 - d["ht"] / f.hs[i] for d in dms]
+        ha.append([(axis((px * c + f.thetax[i] * d["ht"] - d["ox"]) / d["dx"], d["nx"]),
+                    axis((py * c + f.thetay[i] * d["ht"] - d["oy"]) / d["dx"], d["ny"])) for d, c in zip(dms, sc)])
+
+    def sparse(sp, v):
+        c, out = sp.tocoo(), np.zeros(sp.shape[0], LD)
+        np.add.at(out, c.row, c.data.astype(LD) * v[c.col])
+        return out
+
+    w1, s = fit.W1().astype(LD), fit.slaving()
+    nw = fit.NW().astype(LD) if f.nnw else np.zeros((off[-1], 0), LD)
+
+    def apply(a):
+        out = LD(f.tikdiag) * a + nw @ (nw.T @ a) + (0 if s is None else sparse(s, a))
+        for i in range(f.nfit):
+            o = sum(my @ a[off[d]:off[d + 1]].reshape(my.shape[1], -1) @ mx.T for d, (mx, my) in enumerate(ha[i])).ravel()
+            o = LD(f.wt[i]) * (sparse(fit.W0(), o) - w1 * np.sum(w1 * o))
+            for d, (mx, my) in enumerate(ha[i]):
+                out[off[d]:off[d + 1]] += (my.T @ o.reshape(f.fny, f.fnx) @ mx).ravel()
+        return out
+
+    return apply
+
+
+def test_assembled_columns_to_the_last_place():
+    """A column of the assembled FitL (of a unit vector) is its coefficients and
+    the low-rank terms.  With each coefficient right to its last place there are
+    four roundings of at most half a unit (1.11e-16) of an entry: the coefficient,
+    a low-rank product, its weight, their sum.  They are independent, so a
+    column's error stays under sqrt(4) x 1.11e-16 = 2.2e-16 or little above: 3e-16.
+    Coefficients summed in plain 64-bit arithmetic are up to 3.5e-16 off, and
+    every iteration repeats their error."""
+    base = configs.batch_member(15.0, 6, 6)
+    fc = configs.fit_for(base)
+    r = tomo.Recon(configs.with_fit_dirs(base, fc))
+    f = tomo.FitSetup(r, fc)
+    g = tomo.GpuFit(r, f)
+    assert g.info()["assembled"] == 1
+    apply = fit_l_80(r, f)
+    worst = 0.0
+    for j in np.random.default_rng(3).integers(0, f.nact, 24):
+        e = np.zeros(f.nact)
+        e[j] = 1.0
+        want = apply(e.astype(np.longdouble))
+        d = g.L(e) - want
+        worst = max(worst, float(np.sqrt(np.sum(d * d) / np.sum(want * want))))
+    print("assembled columns: worst rel %.2e" % worst, flush=True)
+    assert worst <= 3e-16
+    g.close()
