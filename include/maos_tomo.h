@@ -426,8 +426,8 @@ int  gpu_tomo_autotune(gpu_tomo_t *g, int nsys, int *choice);
  * FFTs in LDS stages, which otherwise run in registers for single-plan
  * batches with layers of 64 or 96 points) and the flights of a
  * graph solve (1, 2, 4, or 0 for 1).  Values above a
- * kernel's maximum (WFS 2 when tomo.pos = 2, column 2 in precision modes 1
- * and 2) are clamped when the launch is built.  Call it before the plan
+ * kernel's maximum (WFS 2 when tomo.pos = 2, column as the LDS holds) are
+ * clamped when the launch is built.  Call it before the plan
  * joins a group.  No reference counterpart. */
 int  gpu_tomo_tune_set(gpu_tomo_t *g, const int *choice);
 

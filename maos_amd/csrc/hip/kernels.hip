@@ -805,7 +805,8 @@ __global__ __launch_bounds__(256) void k_layer(KARGS, int psel_, int osel, int p
 // of layers (k_layer: WFS), a round trip to memory each.  With WS > 1 the
 // workgroup has WS groups of threads that take the layers (WFS) in turn; their
 // terms go to LDS and are added in the order of the loop, so the bits are
-// those of WS = 1.  One 30 m system: k_wfs_m 6.1 -> 5.3, k_layer_m8 7.6 -> 6.2 us.
+// those of WS = 1.  One 30 m system: k_wfs_m 6.6 -> 5.1, k_layer_m 7.4 -> 5.3 us;
+// two: k_layer_m8 on 16 x 32 tiles 8.5 -> 5.9.
 constexpr int WSMAX = 8;  // most layers (WFS) of the split forms
 template <int POS, typename RT, int CS, int WS = 1>
 __global__ __launch_bounds__(256 * WS) void k_wfs_m(KARGS, int xsel) {

@@ -1120,7 +1120,9 @@ void build_stage(Batch &B, Stage &out, KeyF key, GridF grid, SubF fill,
 }
 
 // Launches of at most this many workgroups (one per CU) take the split forms
-// of k_wfs_m (tomo.pos = 1) and the layer kernels.  us per launch, back to back,
+// of k_wfs_m (tomo.pos = 1) and the layer kernels (k_layer_m8's where a launch of
+// few workgroups is on 16 x 32 tiles: two systems of 30 m, or one where 32 rows
+// are set).  us per launch, back to back,
 // whole / split: k_layer_m8 of the 30 m system (108 workgroups each) 1 system
 // 7.6 6.2, 2: 7.6 6.2, 4: 7.8 10.3; k_layer_m of the 20 m one (64) 4: 5.8 5.2, 6:
 // 5.9 6.8; k_wfs_m of the 30 m one (96) 1: 6.1 5.3, 4: 6.7 7.6, of the 20 m one
@@ -1282,9 +1284,10 @@ std::unique_ptr<Batch> make_batch(const std::vector<gpu_tomo *> &plans, const st
         // register kernel where the plan allows it and the tuning does not
         // ask for the LDS kernel (a property of the plan, as for the rows).
         // One plan: a launch per (P, lanes, block size), specialised where an
-        // instantiation exists.  Several plans: one launch per P, the
-        // runtime lanes / block size variant (the same operations in the
-        // same order, so the same bits) with the largest workgroup.
+        // instantiation exists.  Several plans: one launch per P with the
+        // largest workgroup, the runtime block size and the lanes at compile
+        // time only where the plans share them (the same operations in the
+        // same order, so the same bits).
         auto colreg = [&](int j) { return b.plan[j]->colr_ok && b.plan[j]->tune_colfft != 2 ? G(j).shP : 0; };
         std::map<int, int> nthr_of_p;  // merged: largest workgroup per P
         std::map<int, int> lanes_of_p;  // ... and its lanes, 0 where they differ

@@ -177,7 +177,7 @@ class GpuTomo:
         return tuple(ch)
 
     def tune_set(self, wfs, layer, col, layer_rows=0, col_fft=0, flights=0):
-        """gpu_tomo_tune_set: fix the systems per workgroup (0: heuristic),
+        """gpu_tomo_tune_set: fix the systems per workgroup (0: built-in choice),
         the layer tile rows (16, 32, 64; 0: built-in choice), the FFT kernels
         (1 registers where they apply, 2 LDS stages for columns and rows;
         0: as 1) and the
