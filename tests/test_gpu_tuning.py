@@ -89,8 +89,8 @@ def test_tune_set_rejects_bad_choice(large30):
 def test_autotune_replay(large30):
     """The autotuner overwrites slots and picks a choice; replaying that
     choice with tune_set gives the same bits, and the result stays within
-    the rounding of the choice of layer tile shape (the order of the p.Ap
-    partial sums) of the solution before tuning."""
+    the rounding of the choice of column kernel (whose FFTs differ) of the
+    solution before tuning."""
     cfg, r = large30
     grads = _batch(r, cfg, 3)
     g = tomo.GpuTomo(r, nbatch=3, maxit=cfg["maxit"])
